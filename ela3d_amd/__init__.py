@@ -436,7 +436,9 @@ def set_tuning(cfg: Config, block: int, zseg_interior: int, zseg_slab: int, vec:
     other; FP16 storage always updates in place and ignores it); ``fused`` (implies
     ``dbuf``) runs the fused interior step with ``tile``
     cells per workgroup and ``zseg_interior`` planes per segment, its workgroups
-    walking ``strips`` xy strips of tiles (0: the default).  A shape a grid
+    walking ``strips`` xy strips of tiles (0: the default); ``fused=2`` runs the whole
+    grid in one launch per step, ``tile`` threads per workgroup (a 64-lane wave per row
+    of cells and one more for the rows beside them; at most 1024, FP64 512).  A shape a grid
     cannot run (a fused tile that does not fit, FP16 storage with ``fused``) falls
     back to the two-pass schedule when the shot is created."""
     from ._lib import TuningStruct
@@ -444,7 +446,7 @@ def set_tuning(cfg: Config, block: int, zseg_interior: int, zseg_slab: int, vec:
     t = TuningStruct(block=block, zseg_interior=zseg_interior, zseg_slab=zseg_slab, vec=vec,
                      candidates=0, ms_per_step=0.0, block_slab=block_slab, vec_slab=vec_slab,
                      overlap=1 if overlap else 0, merged=1 if merged else 0,
-                     dbuf=1 if (dbuf or fused) else 0, fused=1 if fused else 0, tile=int(tile),
+                     dbuf=1 if (dbuf or fused) else 0, fused=2 if fused == 2 else 1 if fused else 0, tile=int(tile),
                      strips=int(strips))
     check(lib().ela3d_tuning_set(C.byref(s), C.byref(t)))
 

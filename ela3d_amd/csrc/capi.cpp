@@ -373,7 +373,8 @@ int ela3d_source_trace(ela3d_shot* s, double* out, size_t cap)
 
 namespace {
 
-// Checkpoint file: this header, then the shot's device allocation byte for byte.
+// Checkpoint file: this header, then the shot's device allocation byte for byte (without a
+// second field set behind it).
 struct CheckpointHeader {
     char magic[8];
     uint32_t version;
@@ -437,7 +438,8 @@ int ela3d_checkpoint_save(ela3d_shot* s, const char* path)
         h.nstep = p.cfg.nstep;
         h.nrec = p.cfg.nrec;
         h.steps_done = s->impl->steps_done();
-        h.state_bytes = uint64_t(s->impl->device_bytes());
+        s->impl->settle_state();
+        h.state_bytes = uint64_t(s->impl->state_bytes());
         h.fingerprint = fingerprint(p);
         File f;
         f.f = std::fopen(path, "wb");
@@ -469,7 +471,7 @@ int ela3d_checkpoint_load(ela3d_shot* s, const char* path)
         CheckpointHeader h;
         if (std::fread(&h, sizeof(h), 1, f.f) != 1 || std::memcmp(h.magic, kMagic, 8) != 0 || h.version != 1)
             throw Error{ELA3D_E_IO, "not an ela3d checkpoint"};
-        if (h.fingerprint != fingerprint(p) || h.state_bytes != uint64_t(s->impl->device_bytes()) ||
+        if (h.fingerprint != fingerprint(p) || h.state_bytes != uint64_t(s->impl->state_bytes()) ||
             h.steps_done < 0 || h.steps_done > p.cfg.nstep)
             throw Error{ELA3D_E_INVALID, "checkpoint belongs to a different configuration"};
         // a short file is refused before any state is overwritten, so the shot is left as it was

@@ -363,9 +363,9 @@ void check_model(int64_t cells, const float* cp, const float* cs, const float* r
     }
 }
 
-int64_t device_bytes_estimate(const ela3d_config& c, const ShotPlan* plan)
+int64_t device_bytes_estimate(const ela3d_config& c, const ShotPlan* plan, bool one_set)
 {
-    if (plan) return shot_device_bytes(*plan);
+    if (plan) return shot_device_bytes(*plan, one_set);
     const int64_t cells = int64_t(c.nx) * c.ny * c.nz;
     const int e = storage_bytes(c.storage);
     const int w = 2 * c.npoints_pml + 2;

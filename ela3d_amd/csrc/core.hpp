@@ -60,6 +60,8 @@ struct ShotPlan {
     double alg_fused_interior() const {
         return alg_stress_interior + alg_velocity_interior - fused_saving * double(interior_cells);
     }
+    // the whole grid in one fused launch
+    double alg_step_march() const { return alg_step() - fused_saving * double(cells); }
     double alg_step_fused() const { return alg_fused_interior() + alg_stress_slab + alg_velocity_slab; }
 };
 
@@ -88,10 +90,10 @@ ShotPlan make_slab_plan(const ela3d_config& cfg, int k0, int k1, std::vector<int
 PmlAxis make_axis(const ela3d_config& cfg, int axis);
 double wavelet_value(const ela3d_config& cfg, double t0, int it);
 // Device bytes a shot of this config holds (used by admission control).
-int64_t device_bytes_estimate(const ela3d_config& cfg, const ShotPlan* plan);
+int64_t device_bytes_estimate(const ela3d_config& cfg, const ShotPlan* plan, bool one_set = false);
 // Throws ELA3D_E_INVALID unless every cell has finite cp > cs > 0 and rho > 0.
 void check_model(int64_t cells, const float* cp, const float* cs, const float* rho);
 // exact size of the single device allocation a shot of this plan makes
-int64_t shot_device_bytes(const ShotPlan& p);
+int64_t shot_device_bytes(const ShotPlan& p, bool one_set = false);
 
 }  // namespace ela3d

@@ -63,6 +63,39 @@ __device__ __forceinline__ R dt_over(R dt, R r)
         return dt / r;
 }
 
+// The FP32 and FP64 updates write every multiply-add and every plain sum out, so that a cell's
+// new values are the same to the bit in every kernel and schedule that runs it (what the
+// compiler contracts by itself depends on the code around an expression).
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <typename R>
+__device__ __forceinline__ R sum_r(R a, R b)
+{
+#pragma clang fp contract(off)
+    return a + b;
+}
+
+// memory-variable recurrence psi <- b psi + a D;  D <- D/K + psi  (CPU:395-405),
+// with 1/K precomputed per table entry: identical to the division for K = 1
+// (the reference's K_MAX_PML = 1, CPU:75), within one rounding otherwise.
+template <typename R>
+__device__ __forceinline__ R recur(R psi, R a, R b, R Kinv, R& d)
+{
+    const R p = fma_r(a, d, b * psi);
+    d = fma_r(d, Kinv, p);
+    return p;
+}
+
+// dt over the averaged density, to the rounding of the IEEE quotient: the hardware
+// reciprocal, and one Newton correction of the product's residual
+__device__ __forceinline__ float dt_quot(float dt, float r)
+{
+    const float y = __builtin_amdgcn_rcpf(r);
+    const float q = dt * y;
+    return __builtin_fmaf(__builtin_fmaf(-q, r, dt), y, q);
+}
+__device__ __forceinline__ double dt_quot(double dt, double r) { return dt / r; }
+
 // Cell energy terms of the total-energy sum, in the arithmetic type R (FP32
 // storage: FP32, about 1e-7 relative, below the state's own rounding; the sums
 // are FP64).  Kinetic 0.5 rho |v|^2.  Strain energy
@@ -76,18 +109,20 @@ __device__ __forceinline__ R dt_over(R dt, R r)
 template <typename R>
 __device__ __forceinline__ R kinetic_energy(R rho, R vx, R vy, R vz)
 {
-    return ((R)0.5 * rho * vx) * vx + ((R)0.5 * rho * vy) * vy + ((R)0.5 * rho * vz) * vz;
+    const R h = (R)0.5 * rho;
+    return fma_r(h * vx, vx, fma_r(h * vy, vy, (h * vz) * vz));
 }
 template <typename R>
 __device__ __forceinline__ R strain_energy(R rho, R vp, R vs, R sxx, R syy, R szz, R sxy, R sxz, R syz)
 {
-    const R mu = rho * vs * vs, lam = rho * (vp * vp - (R)2 * vs * vs);
-    const R q = (R)3 * lam + (R)2 * mu;
+    const R mu = rho * vs * vs, lam = rho * fma_r(vp, vp, (R)-2 * vs * vs);
+    const R q = fma_r((R)3, lam, (R)2 * mu);
     const R c = (R)1 / ((R)4 * mu * q);
     const R a = q * c, a2 = (R)2 * a, b = lam * c;
     const R tr = sxx + syy + szz;
-    return (a * sxx) * sxx + (a * syy) * syy + (a * szz) * szz +
-           (a2 * sxy) * sxy + (a2 * sxz) * sxz + (a2 * syz) * syz - (b * tr) * tr;
+    const R n = fma_r(a * sxx, sxx, fma_r(a * syy, syy, (a * szz) * szz));
+    const R s = fma_r(a2 * sxy, sxy, fma_r(a2 * sxz, sxz, (a2 * syz) * syz));
+    return fma_r(-(b * tr), tr, n + s);
 }
 
 // Streaming (nontemporal) store of element o of p.  For the nine wave fields: a

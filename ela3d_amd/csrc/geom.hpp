@@ -157,4 +157,39 @@ __host__ __device__ inline int fused_cell(int t, int n, int nx)
 // lines, not three; the threads left over idle.
 __host__ __device__ inline int fused_own(int nt, int nx) { return (nt - 2 * nx) / 32 * 32; }
 
+// Whole-grid fused step (march.hip): tile `chunk` of the plane is the x chunk
+// chunk % xch of the rows of tile chunk / xch.  It owns n rows from j0 and the columns
+// [x0, x1); lanes hold [xs, xe), one column more on each side where the grid goes on.
+struct MarchTile {
+    int j0, n, x0, x1, xs, xe;
+};
+__host__ __device__ inline MarchTile march_tile(int nx, int ny, int rows, int xch, int xw, int chunk)
+{
+    MarchTile t;
+    const int ty = chunk / xch, tx = chunk - ty * xch;
+    t.j0 = ty * rows;
+    t.n = rows < ny - t.j0 ? rows : ny - t.j0;
+    t.x0 = tx * xw;
+    t.x1 = t.x0 + xw < nx ? t.x0 + xw : nx;
+    t.xs = tx > 0 ? t.x0 - 1 : 0;
+    t.xe = t.x1 + 1 < nx ? t.x1 + 1 : nx;
+    return t;
+}
+// Columns per x chunk: the fewest chunks whose columns, halo columns included, fit a wave.
+__host__ __device__ inline int march_chunk_width(int nx, int& xch)
+{
+    for (xch = 1;; ++xch) {
+        const int w = (nx + xch - 1) / xch;
+        if (w + (xch > 2 ? 2 : xch - 1) <= 64) return w;
+    }
+}
+constexpr unsigned kMarchLds = 160 * 1024;  // LDS of a compute unit
+constexpr int kMarchThreads = 1024;         // most threads of a workgroup (FP64: half)
+// LDS of a workgroup: two sets of 8 row buffers of rows + 2 rows, the column tables, and the
+// row and plane tables
+__host__ __device__ inline unsigned march_lds_bytes(int elem, int rows, int zseg)
+{
+    return unsigned((16 * (rows + 2) + 10) * 64 + 6 * (rows + 2 + zseg + 2)) * unsigned(elem);
+}
+
 }  // namespace ela3d

@@ -192,26 +192,37 @@ __device__ __forceinline__ void stv(T* p, unsigned o, const typename Arith<T>::R
 
 // dt over the averaged density in the velocity updates: the reciprocal form
 // (dt_over) with FP16 storage, whose kernels are bound by instruction issue
-// (2.4-2.8 % faster on the layered grid); the IEEE division with FP32 and FP64
-// storage, where the reciprocal measured no faster in these kernels.
+// (2.4-2.8 % faster on the layered grid); the corrected one with FP32 and FP64.
 template <typename T, typename R>
 __device__ __forceinline__ R quot(R dt, R r)
 {
     if constexpr (std::is_same<T, half_t>::value)
         return dt_over(dt, r);
     else
-        return dt / r;
+        return dt_quot(dt, r);
 }
 
-// memory-variable recurrence psi <- b psi + a D;  D <- D/K + psi  (CPU:395-405),
-// with 1/K precomputed per table entry: identical to the division for K = 1
-// (the reference's K_MAX_PML = 1, CPU:75), within one rounding otherwise.
-template <typename R>
-__device__ __forceinline__ R cpml(R psi_old, R a, R b, R Kinv, R& d)
+// a + b: with FP32 and FP64 never contracted with a product (see sum_r); FP16 storage
+// has one schedule only, and the compiler may
+template <typename T, typename R>
+__device__ __forceinline__ R sum(R a, R b)
 {
-    const R psi = b * psi_old + a * d;
-    d = d * Kinv + psi;
-    return psi;
+    if constexpr (std::is_same<T, half_t>::value)
+        return a + b;
+    else
+        return sum_r(a, b);
+}
+
+// acc + d, where d = diff * inv is the derivative along y or z, `layer` saying whether that
+// axis's memory variable has changed it: one fused multiply-add where it has not, in every
+// box and schedule alike (FP16 storage: see sum)
+template <typename T, int MODE, typename R>
+__device__ __forceinline__ R add_axis(R acc, R diff, R inv, R d, bool layer)
+{
+    if constexpr (std::is_same<T, half_t>::value)
+        return acc + d;
+    else
+        return MODE == kSlab && layer ? sum_r(acc, d) : fma_r(diff, inv, acc);
 }
 
 // Element type the x/y C-PML coefficients are read in: the FP32 copies of the
@@ -411,90 +422,93 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
         {
             onN[e] = L.act[e] && (i <= nx - 2) && (j >= 1) && (k >= 1 || surface);
             const R vp = P.cp_c[e];
-            const R lambda = Q.rho_c[e] * (vp * vp - (R)2 * Q.cs_c[e] * Q.cs_c[e]);
+            const R lambda = Q.rho_c[e] * fma_r(vp, vp, (R)-2 * Q.cs_c[e] * Q.cs_c[e]);
             const R l2m = Q.rho_c[e] * vp * vp;
             const R DT_l2m = dt * l2m, DT_l = dt * lambda;
             R dvx_dx = (P.vxE[e] - vx_c) * idx;
             R dvy_dy = (vy_c - P.vyS[e]) * idy;
             R dvz_dz = (P.vz_c[e] - Q.vz_m[e]) * idz;
             if (cx >= 0) {
-                const R m = cpml(P.mx[0][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], dvx_dx);
+                const R m = recur(P.mx[0][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], dvx_dx);
                 if (onN[e]) stm(mout(A, 0), omx, m, S, 9);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = cpml(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], dvy_dy);
+                    const R m = recur(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], dvy_dy);
                     if (onN[e]) stm(mout(A, 1), omy, m, S, 10);
                 }
                 if (Z.cz >= 0) {
-                    const R m = cpml(P.mz[0][e], Z.az, Z.bz, Z.Kz, dvz_dz);
+                    const R m = recur(P.mz[0][e], Z.az, Z.bz, Z.Kz, dvz_dz);
                     if (onN[e]) stm(mout(A, 2), omz, m, S, 11);
                 }
             }
             if (surface) {
                 // traction-free surface (sigma_zz = 0 on plane 0): the vertical strain
                 // rate follows from lambda (exx + eyy) + (lambda + 2 mu) ezz = 0
-                dvz_dz = -(lambda / l2m) * (dvx_dx + dvy_dy);
+                dvz_dz = -(lambda / l2m) * sum<T>(dvx_dx, dvy_dy);
             }
-            nsxx[e] = DT_l2m * dvx_dx + DT_l * (dvy_dy + dvz_dz) + P.sxx[e];
-            nsyy[e] = DT_l * (dvx_dx + dvz_dz) + DT_l2m * dvy_dy + P.syy[e];
-            nszz[e] = surface ? P.szz[e] : DT_l * (dvx_dx + dvy_dy) + DT_l2m * dvz_dz + P.szz[e];
+            nsxx[e] = sum<T>(fma_r(DT_l2m, dvx_dx, DT_l * sum<T>(dvy_dy, dvz_dz)), P.sxx[e]);
+            nsyy[e] = sum<T>(fma_r(DT_l2m, dvy_dy, DT_l * sum<T>(dvx_dx, dvz_dz)), P.syy[e]);
+            nszz[e] = surface ? P.szz[e] : sum<T>(fma_r(DT_l2m, dvz_dz, DT_l * sum<T>(dvx_dx, dvy_dy)), P.szz[e]);
         }
         // sigma_xy: i in [1,nx-1], j in [0,ny-2]; mu averaged over (i-1,j),(i,j+1) (CPU:415-442)
         {
             onXY[e] = L.act[e] && (i >= 1) && (j <= ny - 2);
-            const R vs = (P.csW[e] + P.csN[e]) / (R)2;
-            const R rh = (P.rhoW[e] + P.rhoN[e]) / (R)2;
+            const R vs = sum<T>(P.csW[e], P.csN[e]) / (R)2;
+            const R rh = sum<T>(P.rhoW[e], P.rhoN[e]) / (R)2;
             const R DT_mu = dt * (rh * vs * vs);
             R dvy_dx = (vy_c - P.vyW[e]) * idx;
-            R dvx_dy = (P.vxN[e] - vx_c) * idy;
+            const R ey = P.vxN[e] - vx_c;
+            R dvx_dy = ey * idy;
             if (cx >= 0) {
-                const R m = cpml(P.mx[1][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvy_dx);
+                const R m = recur(P.mx[1][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvy_dx);
                 if (onXY[e]) stm(mout(A, 3), omx, m, S, 12);
             }
             if (MODE == kSlab && cy >= 0) {
-                const R m = cpml(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvx_dy);
+                const R m = recur(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvx_dy);
                 if (onXY[e]) stm(mout(A, 4), omy, m, S, 13);
             }
-            nsxy[e] = DT_mu * (dvy_dx + dvx_dy) + P.sxy[e];
+            nsxy[e] = fma_r(DT_mu, add_axis<T, MODE>(dvy_dx, ey, idy, dvx_dy, cy >= 0), P.sxy[e]);
         }
         // sigma_xz: i in [1,nx-1]; mu averaged over (i-1,k),(i,k+1) (CPU:444-470)
         {
             onXZ[e] = L.act[e] && shear_k && (i >= 1);
-            const R vs = (P.csW[e] + P.cs_u[e]) / (R)2;
-            const R rh = (P.rhoW[e] + P.rho_u[e]) / (R)2;
+            const R vs = sum<T>(P.csW[e], P.cs_u[e]) / (R)2;
+            const R rh = sum<T>(P.rhoW[e], P.rho_u[e]) / (R)2;
             const R DT_mu = dt * (rh * vs * vs);
             R dvz_dx = (P.vz_c[e] - P.vzW[e]) * idx;
-            R dvx_dz = (P.vx_u[e] - vx_c) * idz;
+            const R ez = P.vx_u[e] - vx_c;
+            R dvx_dz = ez * idz;
             if (cx >= 0) {
-                const R m = cpml(P.mx[2][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvz_dx);
+                const R m = recur(P.mx[2][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvz_dx);
                 if (onXZ[e]) stm(mout(A, 5), omx, m, S, 14);
             }
             if (MODE == kSlab && Z.cz >= 0) {
-                const R m = cpml(P.mz[1][e], Z.azh, Z.bzh, Z.Kzh, dvx_dz);
+                const R m = recur(P.mz[1][e], Z.azh, Z.bzh, Z.Kzh, dvx_dz);
                 if (onXZ[e]) stm(mout(A, 6), omz, m, S, 15);
             }
-            nsxz[e] = DT_mu * (dvz_dx + dvx_dz) + P.sxz[e];
+            nsxz[e] = fma_r(DT_mu, add_axis<T, MODE>(dvz_dx, ez, idz, dvx_dz, Z.cz >= 0), P.sxz[e]);
         }
         // sigma_yz: j in [0,ny-2]; mu averaged over (j+1,k),(j,k+1) (CPU:472-497)
         {
             onYZ[e] = L.act[e] && shear_k && (j <= ny - 2);
-            const R vs = (P.csN[e] + P.cs_u[e]) / (R)2;
-            const R rh = (P.rhoN[e] + P.rho_u[e]) / (R)2;
+            const R vs = sum<T>(P.csN[e], P.cs_u[e]) / (R)2;
+            const R rh = sum<T>(P.rhoN[e], P.rho_u[e]) / (R)2;
             const R DT_mu = dt * (rh * vs * vs);
             R dvz_dy = (P.vzN[e] - P.vz_c[e]) * idy;
-            R dvy_dz = (P.vy_u[e] - vy_c) * idz;
+            const R ez = P.vy_u[e] - vy_c;
+            R dvy_dz = ez * idz;
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = cpml(P.my[2][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvz_dy);
+                    const R m = recur(P.my[2][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvz_dy);
                     if (onYZ[e]) stm(mout(A, 7), omy, m, S, 16);
                 }
                 if (Z.cz >= 0) {
-                    const R m = cpml(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, dvy_dz);
+                    const R m = recur(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, dvy_dz);
                     if (onYZ[e]) stm(mout(A, 8), omz, m, S, 17);
                 }
             }
-            nsyz[e] = DT_mu * (dvz_dy + dvy_dz) + P.syz[e];
+            nsyz[e] = fma_r(DT_mu, add_axis<T, MODE>(dvz_dy, ez, idz, dvy_dz, Z.cz >= 0), P.syz[e]);
         }
     }
     if constexpr (Scales<T>::on) {  // the source cell's new normal stresses go to the side slot
@@ -680,79 +694,85 @@ __device__ __forceinline__ void velocity_update(const StepArgs<T>& A, const Lane
         const bool onx = L.act[e] && (i >= 1) && (j >= 1) && (k >= 1 || surface);
         nvx[e] = P.vx[e];
         {
-            const R rh = (Q.rho_c[e] + P.rhoW[e]) / (R)2;
+            const R rh = sum<T>(Q.rho_c[e], P.rhoW[e]) / (R)2;
             const R DT_over_rho = quot<T>(dt, rh);
             R d1 = (P.sxx[e] - P.sxxW[e]) * idx;
-            R d2 = (P.sxy[e] - P.sxyS[e]) * idy;
-            R d3 = (P.sxz[e] - (surface ? -P.sxz[e] : Q.sxz_m[e])) * idz;
+            const R e2 = P.sxy[e] - P.sxyS[e];
+            R d2 = e2 * idy;
+            const R e3 = P.sxz[e] - (surface ? -P.sxz[e] : Q.sxz_m[e]);
+            R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = cpml(P.mx[0][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], d1);
+                const R m = recur(P.mx[0][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], d1);
                 if (onx) stm(mout(A, 9), omx, m, S, 18);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = cpml(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
+                    const R m = recur(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
                     if (onx) stm(mout(A, 10), omy, m, S, 19);
                 }
                 if (Z.cz >= 0) {
-                    const R m = cpml(P.mz[0][e], Z.az, Z.bz, Z.Kz, d3);
+                    const R m = recur(P.mz[0][e], Z.az, Z.bz, Z.Kz, d3);
                     if (onx) stm(mout(A, 11), omz, m, S, 20);
                 }
             }
             if (onx)
-                nvx[e] = DT_over_rho * (d1 + d2 + d3) + P.vx[e];
+                nvx[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vx[e]);
         }
         // vy: i in [0,nx-2], j in [0,ny-2], k in [1,nz-1] (CPU:531-558), plane 0 at a free surface
         const bool ony = L.act[e] && (i <= nx - 2) && (j <= ny - 2) && (k >= 1 || surface);
         nvy[e] = P.vy[e];
         {
-            const R rh = (Q.rho_c[e] + P.rhoN[e]) / (R)2;
+            const R rh = sum<T>(Q.rho_c[e], P.rhoN[e]) / (R)2;
             const R DT_over_rho = quot<T>(dt, rh);
             R d1 = (P.sxyE[e] - P.sxy[e]) * idx;
-            R d2 = (P.syyN[e] - P.syy[e]) * idy;
-            R d3 = (P.syz[e] - (surface ? -P.syz[e] : Q.syz_m[e])) * idz;
+            const R e2 = P.syyN[e] - P.syy[e];
+            R d2 = e2 * idy;
+            const R e3 = P.syz[e] - (surface ? -P.syz[e] : Q.syz_m[e]);
+            R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = cpml(P.mx[1][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
+                const R m = recur(P.mx[1][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
                 if (ony) stm(mout(A, 12), omx, m, S, 21);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = cpml(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], d2);
+                    const R m = recur(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], d2);
                     if (ony) stm(mout(A, 13), omy, m, S, 22);
                 }
                 if (Z.cz >= 0) {
-                    const R m = cpml(P.mz[1][e], Z.az, Z.bz, Z.Kz, d3);
+                    const R m = recur(P.mz[1][e], Z.az, Z.bz, Z.Kz, d3);
                     if (ony) stm(mout(A, 14), omz, m, S, 23);
                 }
             }
             if (ony)
-                nvy[e] = DT_over_rho * (d1 + d2 + d3) + P.vy[e];
+                nvy[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vy[e]);
         }
         // vz: i in [0,nx-2], j in [1,ny-1], k in [0,nz-2] (CPU:562-590)
         const bool onz = L.act[e] && (i <= nx - 2) && (j >= 1) && (k <= nz - 2);
         nvz[e] = P.vz[e];
         {
-            const R rh = (Q.rho_c[e] + P.rho_u[e]) / (R)2;
+            const R rh = sum<T>(Q.rho_c[e], P.rho_u[e]) / (R)2;
             const R DT_over_rho = quot<T>(dt, rh);
             R d1 = (P.sxzE[e] - P.sxz[e]) * idx;
-            R d2 = (P.syz[e] - P.syzS[e]) * idy;
-            R d3 = (P.szz_u[e] - Q.szz_c[e]) * idz;
+            const R e2 = P.syz[e] - P.syzS[e];
+            R d2 = e2 * idy;
+            const R e3 = P.szz_u[e] - Q.szz_c[e];
+            R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = cpml(P.mx[2][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
+                const R m = recur(P.mx[2][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
                 if (onz) stm(mout(A, 15), omx, m, S, 24);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = cpml(P.my[2][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
+                    const R m = recur(P.my[2][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
                     if (onz) stm(mout(A, 16), omy, m, S, 25);
                 }
                 if (Z.cz >= 0) {
-                    const R m = cpml(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, d3);
+                    const R m = recur(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, d3);
                     if (onz) stm(mout(A, 17), omz, m, S, 26);
                 }
             }
             if (onz)
-                nvz[e] = DT_over_rho * (d1 + d2 + d3) + P.vz[e];
+                nvz[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vz[e]);
         }
         // rigid faces: the memory variables above are still advanced, then v = 0
         const bool f = face && L.act[e];

@@ -13,6 +13,7 @@ constexpr int kInterior = 0;  // y and z outside the C-PML: only x is checked pe
 constexpr int kSlab = 1;      // y or z inside the C-PML: every axis checked
 constexpr int kMixed = 2;     // launch mode only: boxes of both kinds, each block runs its box's body
 constexpr int kFused = 3;     // launch mode only: one fused stress+velocity step over the interior box
+constexpr int kMarch = 4;     // launch mode only: one fused step over the whole grid
 
 // FP16 storage keeps one power-of-two scale per field (stored = value * scale)
 // in a device table of kScaleTable floats, so replayed graphs see live values:
@@ -84,6 +85,8 @@ struct StepArgs {
     unsigned fdin, fdout, mdin, mdout;
     int tile;                // kFused: threads per workgroup = region cells (own cells + 2 halo rows)
     int ldsreg;              // kFused: cells of one LDS stress plane (= tile)
+    int rows;                // kMarch: rows a workgroup owns
+    int xch, xw;             // kMarch: x chunks, and the columns each owns
 };
 
 template <typename T>
@@ -130,6 +133,10 @@ void launch_fused(const StepArgs<T>& a, bool energy, hipStream_t s);
 // multiple of 64 in [64, max], or fewer than 64 own cells)
 template <typename T>
 size_t fused_lds_bytes(int nx, int tile);
+// fused step over the whole grid, absorbing layers included (march.hip); needs
+// double-buffered fields.  A workgroup has a wave per own row and two halo waves.
+template <typename T>
+void launch_march(const StepArgs<T>& a, bool energy, hipStream_t s);
 template <typename T>
 void launch_tail(const TailArgs<T>& a, hipStream_t s);
 // A batch of shots stepped together (each a merged launch over all its boxes,

@@ -122,6 +122,7 @@ struct Request {
     std::vector<int32_t> rec;
     std::vector<float> cp, cs, rho;
     int64_t bytes = 0;           // device bytes charged to the budget
+    bool one_set = false;        // steps in place unless its launch shape was measured or given
     std::atomic<int> state{ELA3D_SHOT_QUEUED};
     std::atomic<int> status{ELA3D_OK};
     double t_submit = 0, t_admit = 0, t_done = 0;
@@ -180,6 +181,13 @@ public:
 
     bool batching() const { return !opts_.plain_loop && opts_.batch_cells > 0 && opts_.max_active > 1; }
 
+    // whether a shot is of the kind that advances in batch launches
+    bool batchable(const ShotPlan& p) const
+    {
+        return batching() && p.cells <= int64_t(opts_.batch_cells) && p.cfg.storage == ELA3D_STORAGE_FP32 &&
+               p.cfg.energy_every <= 0;
+    }
+
     void free_slots()
     {
         (void)hipSetDevice(opts_.device);
@@ -216,7 +224,10 @@ public:
         r->cp.assign(cp, cp + n);
         r->cs.assign(cs, cs + n);
         r->rho.assign(rho, rho + n);
-        r->bytes = device_bytes_estimate(plan.cfg, &plan);
+        // Shots for the batch launches update in place, and so does one whose second field set
+        // would not fit the budget.
+        r->one_set = batchable(plan) || device_bytes_estimate(plan.cfg, &plan) > opts_.hbm_budget_bytes;
+        r->bytes = device_bytes_estimate(plan.cfg, &plan, r->one_set);
         r->nsamples = plan.nsamples;
         r->nenergy = plan.nenergy;
         if (r->bytes > opts_.hbm_budget_bytes)
@@ -381,7 +392,7 @@ private:
                 c.device = opts_.device;
                 return c;
             }());
-            const size_t need = size_t(shot_device_bytes(plan));
+            const size_t need = size_t(shot_device_bytes(plan, r->one_set));
             for (size_t q = 0; q < slots_.size(); ++q)
                 if (!slots_[q].busy) {
                     r->slot = int(q);
@@ -395,6 +406,7 @@ private:
             mem.arena = r->mem;
             mem.bytes = need;
             mem.host_flag = sl.flag;
+            mem.one_set = r->one_set;
             r->shot = make_shot(std::move(plan), r->cp.data(), r->cs.data(), r->rho.data(), sl.stream, false, mem);
             const int64_t actual = r->shot->device_bytes();
             {

@@ -59,11 +59,62 @@ void device_free(void* p, size_t bytes)
     g_device_held -= int64_t(bytes);
 }
 
-Tuning choose_tuning(const ShotPlan& p)
+// Last-level cache in front of HBM
+constexpr int64_t kInfinityCache = int64_t(256) << 20;
+
+// The whole-grid fused step (march.hip) as the schedule of a new shot, in place of two passes.
+// It reads and writes every array once per step (two passes: about 1.6 times the bytes) but
+// keeps two field sets and, with few columns per wave, idles lanes.  Measured, us per step,
+// two passes against one launch:
+//  * launch-bound and small grids: 33^3 30 -> 19, 64^3 33 -> 24, 101^3 51 -> 43;
+//  * beyond the 256 MiB cache: 201^3 261 -> 253, 256^3 490 -> 446, 401x401x301 1311 -> 1200,
+//    480x500x360 2252 -> 2030, FP64 192x200x188 424 -> 379;
+//  * where one set stays in the cache and two do not, two passes stay ahead: 144^3 93 / 119,
+//    160^3 115 / 145, 170^3 156 / 171, FP64 120^3 101 / 126 (at 180^3, one set 1.2 times the
+//    cache, both take the same);
+//  * with more workgroups than fit at once and fewer than 0.6 of a wave's lanes on columns, the
+//    lanes decide: 65x800x640 (0.51) 1013 / 1091, 72x800x640 (0.56) 1095 / 1122, 80x800x640
+//    (0.63) 1195 / 1145, 130x600x640 (0.68) 1425 / 1403.
+// The second set also has to be a small part of the memory: 16 of 288 GB for both.
+static bool march_by_rule(const ShotPlan& p, Tuning& t)
+{
+    const ela3d_config& c = p.cfg;
+    if (c.storage == ELA3D_STORAGE_FP16) return false;
+    const bool dbl = c.storage == ELA3D_STORAGE_FP64;
+    Tuning m = t;
+    m.fused = 2;
+    m.dbuf = 1;
+    // Workgroup: short ones (3 rows and the halo wave) balance best over the grids measured; FP64
+    // has registers for half as many waves and more halo arithmetic per row, so 7 rows.
+    m.tile = dbl ? 512 : 256;
+    m.strips = 4;
+    // z segment: the shortest whose workgroups are all on the chip at once (24 waves per compute
+    // unit, FP64 16); at most 6 planes, where the planes reloaded at a segment's ends cost less
+    // than the imbalance of longer ones (401x401x301: 4 / 6 / 8 planes 1195 / 1203 / 1242 us,
+    // 256^3: 457 / 446 / 458).
+    int xch = 0;
+    const int xw = march_chunk_width(c.nx, xch), rows = m.tile / 64 - 1;
+    const int64_t tiles = int64_t((c.ny + rows - 1) / rows) * xch, fit = int64_t(256) * (dbl ? 16 : 24) * 64 / m.tile;
+    int z = 1;
+    while (z < 6 && tiles * ((c.nz + z - 1) / z) > fit) ++z;
+    m.zseg_interior = z;
+    if (!march_unsupported(p, m).empty()) return false;
+    if (tiles * ((c.nz + z - 1) / z) > fit && c.nx * 10 < xch * 64 * 6) return false;
+    const int elem = storage_bytes(c.storage);
+    const int64_t one = int64_t(arena_layout(p, elem, 0, kOneSet).total);
+    const int64_t two = int64_t(arena_layout(p, elem, 0, kSetAppended).total);
+    if (two > (int64_t(16) << 30)) return false;
+    if (two > kInfinityCache && one < kInfinityCache / 4 * 5) return false;
+    t = m;
+    return true;
+}
+
+Tuning choose_tuning(const ShotPlan& p, bool one_set)
 {
     Tuning t;
     const ela3d_config& c = p.cfg;
     if (c.block == 0 && c.zseg == 0 && cached_tuning(c, t)) return t;
+    t.rule = 1;
     t.block = c.block > 0 ? c.block : 256;
     t.block_slab = t.block;
     t.vec = 1;
@@ -81,6 +132,7 @@ Tuning choose_tuning(const ShotPlan& p)
     while (zs > 2 && nchunk * ((nzi + zs - 1) / zs) < 8192) zs /= 2;
     t.zseg_interior = zs;
     t.zseg_slab = 4;
+    if (!one_set && c.block == 0) march_by_rule(p, t);
     return t;
 }
 
@@ -116,6 +168,23 @@ void geometry(const ShotPlan& p, const Tuning& t, LaunchGeom& slab, LaunchGeom& 
     interior.block = t.block;
     interior.vec = t.vec;
     interior.mode = t.fused ? kFused : t.merged ? kMixed : kInterior;
+    if (t.fused == 2) {  // one launch over the whole grid, one workgroup per (rows x x chunk, z segment)
+        interior.mode = kMarch;
+        interior.block = t.tile;
+        interior.tile = t.tile;
+        interior.rows = t.tile / 64 - 1;
+        interior.vec = 1;
+        interior.xw = march_chunk_width(p.cfg.nx, interior.xch);
+        Box& b = interior.box[interior.nbox++];
+        b.p0 = 0; b.p1 = p.cfg.nx * p.cfg.ny; b.k0 = 0; b.k1 = p.cfg.nz;
+        b.nchunk = (p.cfg.ny + interior.rows - 1) / interior.rows * interior.xch;
+        b.zseg = std::max(1, t.zseg_interior);
+        b.blk0 = 0;
+        b.mode = kMarch;
+        b.nstrip = std::max(0, std::min(t.strips, b.nchunk));
+        interior.nblocks = b.nchunk * ((b.k1 - b.k0 + b.zseg - 1) / b.zseg);
+        return;
+    }
     if (t.fused) {  // one workgroup per (tile, z segment): `tile` threads, one per region cell
         interior.block = t.tile;
         interior.vec = 1;
@@ -176,6 +245,28 @@ std::string fused_unsupported(const ShotPlan& p, int tile)
     return "the grid has no interior box";
 }
 
+static int epart_capacity(const ela3d_config& c)
+{
+    return int((plane_stride(c.nx, c.ny) / 64 + kMaxBox + 1) * int64_t(c.nz) + 8);
+}
+
+std::string march_unsupported(const ShotPlan& p, const Tuning& t)
+{
+    const ela3d_config& c = p.cfg;
+    if (c.storage == ELA3D_STORAGE_FP16) return "the whole-grid fused schedule runs FP32 and FP64 storage only";
+    if (p.koff != 0 || p.own_k0 != 0 || p.own_k1 != c.nz || p.nz_global != c.nz)
+        return "the whole-grid fused schedule does not run z-slabs";
+    const int elem = c.storage == ELA3D_STORAGE_FP64 ? 8 : 4;
+    const int most = kMarchThreads / (elem / 4);
+    if (t.tile % 64 != 0 || t.tile < 128 || t.tile > most)
+        return "threads per workgroup must be a multiple of 64, at least 128 and at most 1024 (512 in FP64)";
+    if (march_lds_bytes(elem, t.tile / 64 - 1, std::max(1, t.zseg_interior)) > kMarchLds) return "the row buffers do not fit the LDS";
+    LaunchGeom slab, all;
+    geometry(p, t, slab, all);
+    if (all.nblocks > epart_capacity(c)) return "too many workgroups for the energy partials";
+    return "";
+}
+
 static size_t mem_elems(const ShotPlan& p, int axis)
 {
     const ela3d_config& c = p.cfg;
@@ -188,8 +279,9 @@ static size_t mem_elems(const ShotPlan& p, int axis)
 // Byte offsets of every buffer in a shot's single device allocation.  Each
 // buffer starts on a 256-byte boundary; the energy-partial buffer has room for
 // any launch shape the tuner may pick (block >= 64, vec >= 1, zseg >= 1).
-ArenaLayout arena_layout(const ShotPlan& p, int elem, int nepart, bool dbuf)
+ArenaLayout arena_layout(const ShotPlan& p, int elem, int nepart, Sets sets)
 {
+    const bool dbuf = sets == kTwoSets;
     const ela3d_config& c = p.cfg;
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
     ArenaLayout L;
@@ -219,7 +311,7 @@ ArenaLayout arena_layout(const ShotPlan& p, int elem, int nepart, bool dbuf)
     const size_t nseis = size_t(p.nsamples) * c.nrec * 3;
     L.seis = off; off += al(std::max<size_t>(1, nseis) * sizeof(double));
     L.energy = off; off += al(std::max<size_t>(1, size_t(p.nenergy) * 2) * sizeof(double));
-    L.epart_cap = int((nxyp / 64 + kMaxBox + 1) * int64_t(c.nz) + 8);
+    L.epart_cap = epart_capacity(c);
     L.epart = off; off += al(size_t(std::max(L.epart_cap, nepart)) * 2 * sizeof(double));
     L.epart2 = off; off += al(size_t(kEpartBlocks) * 2 * sizeof(double));
     L.ctl = off; off += al(2 * sizeof(int));
@@ -228,21 +320,29 @@ ArenaLayout arena_layout(const ShotPlan& p, int elem, int nepart, bool dbuf)
     L.srctrace = off; off += al((size_t(c.nstep) + 1) * 3 * sizeof(double));
     L.tabf = off; off += al(6 * size_t(c.nx + c.ny) * sizeof(float));
     L.side = off; off += al(3 * sizeof(float));
+    L.state = off;
+    if (sets == kSetAppended) {
+        for (int q = 0; q < 9; ++q) { L.f2[q] = off; off += al(padded * elem); }
+        for (int q = 0; q < 18; ++q) { L.m2[q] = off; off += al(mem_elems(p, kMemAxis[q]) * elem); }
+    }
     L.total = off;
     return L;
 }
 
-// FP16 storage always updates in place: its kernels store through the input
-// pointers, and it has no fused schedule, the one that needs two field sets.
-static bool double_buffers(const ShotPlan& p, bool asked)
+// Field sets of a shot with launch shape t (asked: two whatever the shape).  FP16 storage
+// always updates in place: its kernels store through the input pointers, and it has no
+// fused schedule.
+static Sets sets_of(const ShotPlan& p, const Tuning& t, bool asked)
 {
-    return asked && p.cfg.storage != ELA3D_STORAGE_FP16;
+    if (p.cfg.storage == ELA3D_STORAGE_FP16) return kOneSet;
+    if (asked || t.fused == 1 || (t.dbuf && t.fused != 2)) return kTwoSets;
+    return t.fused == 2 ? kSetAppended : kOneSet;
 }
 
-int64_t shot_device_bytes(const ShotPlan& p)
+int64_t shot_device_bytes(const ShotPlan& p, bool one_set)
 {
-    const Tuning t = choose_tuning(p);
-    return int64_t(arena_layout(p, storage_bytes(p.cfg.storage), 0, double_buffers(p, t.dbuf != 0)).total);
+    const Tuning t = choose_tuning(p, one_set);
+    return int64_t(arena_layout(p, storage_bytes(p.cfg.storage), 0, sets_of(p, t, false)).total);
 }
 
 template <typename T>
@@ -276,23 +376,38 @@ private:
             HIP_CHECK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
             own_stream_ = true;
         }
-        tune_ = choose_tuning(plan_);
-        if (tune_.fused && !fused_unsupported(plan_, tune_.tile).empty()) tune_.fused = 0;
+        tune_ = choose_tuning(plan_, mem_.inplace || mem_.one_set);
+        if (tune_.fused == 1 && !fused_unsupported(plan_, tune_.tile).empty()) tune_.fused = 0;
+        if (tune_.fused == 2 && !march_unsupported(plan_, tune_).empty()) tune_.fused = 0;
         if (mem_.inplace) {
             tune_.fused = 0;
             tune_.dbuf = 0;
             tune_.overlap = 0;
             dbuf = false;
         }
-        dbuf_ = double_buffers(plan_, dbuf || tune_.dbuf != 0 || tune_.fused != 0);
-        tune_.dbuf = dbuf_ ? 1 : 0;
-        overlap_ = tune_.overlap != 0;
+        set_shape(dbuf);
         if (overlap_) make_aux();
-        geometry(plan_, tune_, geo_[1], geo_[0]);
-        allocate();
+        try {
+            allocate();
+        } catch (const Error& e) {  // no room for the second set of a schedule taken by rule
+            if (e.code != ELA3D_E_OOM || !tune_.rule || !dbuf_ || dbuf) throw;
+            tune_ = choose_tuning(plan_, true);
+            set_shape(false);
+            allocate();
+        }
         upload(cp, cs, rho);
         initial_scales(cp, rho);
         set_args();
+    }
+
+    // sets, overlap and geometry of tune_
+    void set_shape(bool asked)
+    {
+        sets_ = sets_of(plan_, tune_, asked);
+        dbuf_ = sets_ != kOneSet;
+        tune_.dbuf = dbuf_ ? 1 : 0;
+        overlap_ = tune_.overlap != 0;
+        geometry(plan_, tune_, geo_[1], geo_[0]);
     }
 
     void release()
@@ -329,6 +444,7 @@ public:
     void enqueue_phase(int phase) override
     {
         HIP_CHECK(hipSetDevice(device_));
+        if (tune_.rule && sets_ == kSetAppended && dbuf_) leave_second_set();
         if (tune_.fused || dbuf_ || overlap_)
             throw Error{ELA3D_E_STATE, "stepping by phases needs the in-place two-pass schedule"};
         const int it = host_step_ + 1;
@@ -341,11 +457,43 @@ public:
             launch_velocity(args_[0][0][1], e, stream_);
             if (e) launch_epart(d_epart_, nepart_, d_epart2_, epart_blocks(), stream_);
             launch_tail(tail_args(0), stream_);
-            host_step_ = it;
+            step_enqueued(it);
         } else {
             throw Error{ELA3D_E_INVALID, "phase must be 0 (stress pass) or 1 (velocity pass and tail)"};
         }
         HIP_CHECK(hipGetLastError());
+    }
+
+    // move the state into the first set (on the stream); the sets' roles start over from there
+    void to_first_set()
+    {
+        if (cur() == 0) return;
+        const ArenaLayout L = arena_layout(plan_, int(sizeof(T)), nepart_, sets_);
+        char* b = static_cast<char*>(arena_);
+        for (int q = 0; q < 9; ++q) {
+            const size_t n = (size_t(nxyp_) * plan_.cfg.nz + 2 * size_t(guard_)) * sizeof(T);
+            HIP_CHECK(hipMemcpyAsync(b + L.f[q], b + L.f2[q], n, hipMemcpyDeviceToDevice, stream_));
+        }
+        for (int q = 0; q < 18; ++q) {
+            const size_t n = mem_elems(plan_, kMemAxis[q]) * sizeof(T);
+            if (n) HIP_CHECK(hipMemcpyAsync(b + L.m[q], b + L.m2[q], n, hipMemcpyDeviceToDevice, stream_));
+        }
+        par_ = 0;
+    }
+
+    // From a schedule with two sets that was taken by rule to two passes in place: for calls
+    // that only those serve.  The second set stays allocated, unused.
+    void leave_second_set()
+    {
+        to_first_set();
+        tune_ = choose_tuning(plan_, true);
+        dbuf_ = false;
+        for (int q = 0; q < 9; ++q) d_f_[1][q] = d_f_[0][q];
+        for (int q = 0; q < 18; ++q) d_m_[1][q] = d_m_[0][q];
+        geometry(plan_, tune_, geo_[1], geo_[0]);
+        nepart_ = geo_[0].nblocks + geo_[1].nblocks;
+        set_args();
+        drop_graphs();
     }
 
     // fields that cross a z interface after `phase`, sent towards higher k (up) or lower k
@@ -406,6 +554,13 @@ public:
         HIP_CHECK(hipGetLastError());
     }
     int64_t device_bytes() const override { return arena_bytes_; }
+    int64_t state_bytes() const override { return state_bytes_; }
+    // an appended second set is no part of a checkpoint
+    void settle_state() override
+    {
+        HIP_CHECK(hipSetDevice(device_));
+        if (sets_ == kSetAppended && dbuf_) to_first_set();
+    }
 
     // one step the production way: a replay of its captured graph (captured on
     // first use), or eager launches when graphs are off
@@ -421,7 +576,7 @@ public:
         } else {
             launch_step(e, nullptr, par);
         }
-        host_step_ = it;
+        step_enqueued(it);
     }
 
     void enqueue_steps(int n) override
@@ -449,7 +604,7 @@ public:
                                          hipMemcpyDeviceToHost, stream_));
                 HIP_CHECK(hipStreamSynchronize(stream_));
             }
-            host_step_ = it;
+            step_enqueued(it);
         }
         HIP_CHECK(hipStreamSynchronize(stream_));
     }
@@ -545,7 +700,11 @@ public:
         HIP_CHECK(hipMemcpy(static_cast<char*>(arena_) + offset, host, bytes, hipMemcpyHostToDevice));
     }
 
-    void set_steps_done(int n) override { host_step_ = n; }
+    void set_steps_done(int n) override
+    {
+        host_step_ = n;
+        par_ = sets_ == kTwoSets ? n & 1 : 0;  // an appended set's state is restored to the first
+    }
 
     void snapshot(int field, double* out) override
     {
@@ -624,7 +783,8 @@ public:
                                                "velocity_interior", "tail"};
         static const char* merged[kLaunches] = {"stress_cpml", "stress", "velocity_cpml", "velocity", "tail"};
         static const char* fused[kLaunches] = {"stress_cpml", "fused_interior", "velocity_cpml", "-", "tail"};
-        const char* const* names = tune_.fused ? fused : tune_.merged ? merged : split;
+        static const char* whole[kLaunches] = {"-", "fused_grid", "-", "-", "tail"};
+        const char* const* names = tune_.fused == 2 ? whole : tune_.fused ? fused : tune_.merged ? merged : split;
         st.assign(kLaunches, ela3d_kernel_stats());
         for (int q = 0; q < kLaunches; ++q) {
             std::snprintf(st[q].name, sizeof(st[q].name), "%s", names[q]);
@@ -637,7 +797,10 @@ public:
         st[2].alg_bytes_per_launch = m ? 0.0 : plan_.alg_velocity_slab;
         st[3].alg_bytes_per_launch = plan_.alg_velocity_interior + (m ? plan_.alg_velocity_slab : 0.0);
         st[4].alg_bytes_per_launch = 0;
-        if (tune_.fused) {
+        if (tune_.fused == 2) {
+            st[0].alg_bytes_per_launch = st[2].alg_bytes_per_launch = st[3].alg_bytes_per_launch = 0;
+            st[1].alg_bytes_per_launch = plan_.alg_step_march();
+        } else if (tune_.fused) {
             st[1].alg_bytes_per_launch = plan_.alg_fused_interior();
             st[3].alg_bytes_per_launch = 0;
         }
@@ -660,7 +823,7 @@ public:
                 if (done % every == 0) {
                     const int it = host_step_ + 1;
                     launch_step(energy_step(it), &ev[size_t(m) * E], cur());
-                    host_step_ = it;
+                    step_enqueued(it);
                     ++m;
                 } else {
                     graph_step();
@@ -690,13 +853,15 @@ public:
 
     void retune(const Tuning& t) override
     {
+        if (sets_ == kSetAppended && t.fused == 1)
+            throw Error{ELA3D_E_INVALID, "the fused interior step needs both sets of an array side by side"};
         HIP_CHECK(hipSetDevice(device_));
         HIP_CHECK(hipStreamSynchronize(stream_));
         if ((t.dbuf != 0 || t.fused != 0) && !dbuf_)
             throw Error{ELA3D_E_INVALID, "double buffering is fixed when the shot is created"};
         if (t.overlap != 0 && mem_.inplace) throw Error{ELA3D_E_INVALID, "this shot runs its launches in sequence"};
         if (t.fused) {
-            const std::string why = fused_unsupported(plan_, t.tile);
+            const std::string why = t.fused == 2 ? march_unsupported(plan_, t) : fused_unsupported(plan_, t.tile);
             if (!why.empty()) throw Error{ELA3D_E_INVALID, why};
         }
         LaunchGeom g[2];
@@ -728,7 +893,7 @@ public:
         std::memset(&o, 0, sizeof(o));
         o.cells = plan_.cells;
         o.device_bytes = arena_bytes_;
-        o.alg_bytes_per_step = tune_.fused ? plan_.alg_step_fused() : plan_.alg_step();
+        o.alg_bytes_per_step = tune_.fused == 2 ? plan_.alg_step_march() : tune_.fused ? plan_.alg_step_fused() : plan_.alg_step();
         o.alg_bytes_stress = plan_.alg_stress_interior + plan_.alg_stress_slab;
         o.alg_bytes_velocity = plan_.alg_velocity_interior + plan_.alg_velocity_slab;
         o.pml_bytes_per_step = plan_.alg_pml;
@@ -802,7 +967,7 @@ private:
         nxyp_ = plane_stride(c.nx, c.ny);
         guard_ = guard_elems(c.nx);
         nepart_ = geo_[0].nblocks + geo_[1].nblocks;
-        const ArenaLayout L = arena_layout(plan_, int(sizeof(T)), nepart_, dbuf_);
+        const ArenaLayout L = arena_layout(plan_, int(sizeof(T)), nepart_, sets_);
         epart_cap_ = L.epart_cap;
         const size_t off = L.total;
         const size_t* o_f = L.f;
@@ -812,6 +977,7 @@ private:
         const size_t o_wav = L.wav, o_rec = L.rec, o_seis = L.seis, o_en = L.energy, o_ep = L.epart;
         const size_t o_ctl = L.ctl, o_scl = L.scl, o_slot = L.slot, o_src = L.srctrace;
         arena_bytes_ = int64_t(off);
+        state_bytes_ = int64_t(L.state);
         if (mem_.arena) {
             if (off > mem_.bytes)
                 throw Error{ELA3D_E_RANGE, "shot needs " + std::to_string(off) + " bytes of device memory, " +
@@ -1007,6 +1173,9 @@ private:
         a.mode = g.mode;
         a.tile = g.tile;
         a.ldsreg = g.tile;
+        a.rows = g.rows;
+        a.xch = g.xch;
+        a.xw = g.xw;
         return a;
     }
 
@@ -1082,6 +1251,19 @@ private:
         auto mark = [&](int q, hipStream_t s) {
             if (ev) HIP_CHECK(hipEventRecord(ev[q], s));
         };
+        if (tune_.fused == 2) {  // everything in one launch
+            for (int q = 0; q < 2; ++q) mark(q, stream_);
+            mark(2, stream_);
+            if constexpr (std::is_same<T, half_t>::value)
+                throw Error{ELA3D_E_INVALID, "the fused schedule does not run FP16 storage"};
+            else
+                launch_march(args_[par][0][0], energy, stream_);
+            for (int q = 3; q < 9; ++q) mark(q, stream_);
+            if (energy) launch_epart(d_epart_, nepart_, d_epart2_, epart_blocks(), stream_);
+            launch_tail(tail_args(par), stream_);
+            mark(9, stream_);
+            return;
+        }
         if (tune_.fused) {  // layers' stresses, the fused interior step, layers' velocities
             mark(0, stream_);
             launch_stress(args_[par][1][0], stream_);
@@ -1174,7 +1356,12 @@ private:
     T* d_m_[2][18] = {};
     bool dbuf_ = false;
     // set holding the current state: steps alternate sets when double buffered
-    int cur() const { return dbuf_ ? (host_step_ & 1) : 0; }
+    int cur() const { return dbuf_ ? par_ : 0; }
+    void step_enqueued(int it)
+    {
+        host_step_ = it;
+        par_ ^= 1;
+    }
     float* d_model_[3] = {};
     double* d_tab_[3] = {};
     double *d_wav_ = nullptr, *d_seis_ = nullptr, *d_energy_ = nullptr, *d_epart_ = nullptr;
@@ -1183,6 +1370,9 @@ private:
     int nepart_ = 0, epart_cap_ = 0;
     int64_t nxyp_ = 0, guard_ = 0;
     int host_step_ = 0;
+    int par_ = 0;            // set that holds the state, when double buffered
+    Sets sets_ = kOneSet;    // of the allocation
+    int64_t state_bytes_ = 0;
     int* h_flag_ = nullptr;  // pinned mirror of d_flag_ (serving)
     double* d_srctrace_ = nullptr;   // [nstep+1][3]
     float* d_tabf_ = nullptr;        // FP32 x and y tables [6][nx], [6][ny]

@@ -27,6 +27,7 @@ struct LaunchGeom {
     int nbox = 0, nblocks = 0, block = 256, vec = 1;
     int mode = kInterior;  // kInterior, kSlab, kMixed or kFused
     int tile = 0;          // kFused: cells per workgroup
+    int rows = 0, xch = 0, xw = 0;  // kMarch: own rows per workgroup, x chunks, columns of one
 };
 
 // Launch tuning chosen for a grid (see tune.cpp): the interior launch and the
@@ -44,8 +45,12 @@ struct Tuning {
     int dbuf = 0;           // 1: two field sets, each step reads one and writes the other
     int fused = 0;          // 1: one fused stress+velocity launch over the interior box
                             //    (needs dbuf; zseg_interior planes per workgroup)
-    int tile = 1024;        // fused: interior cells of the flattened plane per workgroup
+                            // 2: one fused launch over the whole grid (needs dbuf;
+                            //    zseg_interior planes per workgroup)
+    int tile = 1024;        // fused: interior cells of the flattened plane per workgroup (1);
+                            //    threads per workgroup, a wave per own row and two more (2)
     int strips = 0;         // fused: xy strips of the tile order (0: the default of tile_of)
+    int rule = 0;           // 1: chosen by choose_tuning's rules, not measured or given
 };
 
 // Device layout of the 9 fields and the 3 model arrays: planes of plane_stride
@@ -55,10 +60,16 @@ int64_t guard_elems(int nx);
 
 struct ArenaLayout {
     size_t f[9], m[18], f2[9], m2[18], model[3], tab[3];
-    size_t wav, rec, seis, energy, epart, epart2, ctl, scl, slot, srctrace, tabf, side, total;
+    size_t wav, rec, seis, energy, epart, epart2, ctl, scl, slot, srctrace, tabf, side;
+    size_t state;  // bytes of a checkpoint: all of it, or up to an appended second set
+    size_t total;
     int epart_cap;
 };
-ArenaLayout arena_layout(const ShotPlan& p, int elem_bytes, int nepart, bool dbuf);
+// Field sets of a shot: one; two, each array's second copy right after its first (the fused
+// interior step addresses both from one base); or two, the second behind everything else, so
+// that what comes before it is the layout of one set (the whole-grid fused step).
+enum Sets { kOneSet = 0, kTwoSets = 1, kSetAppended = 2 };
+ArenaLayout arena_layout(const ShotPlan& p, int elem_bytes, int nepart, Sets sets);
 
 // A shot's share of a batch launch (FP32 storage, in place, no energy sums):
 // its merged-launch arguments for both passes, its tail, and its block count.
@@ -89,7 +100,10 @@ public:
     virtual void energy(double* out) = 0;           // nenergy*2
     virtual void source_trace(double* out) = 0;     // (nstep+1)*3
     // raw access to the whole device state (every buffer of the single allocation,
-    // device_bytes() long) for checkpoints; set_steps_done after a full restore
+    // state_bytes() long) for checkpoints, after settle_state; set_steps_done after a
+    // full restore
+    virtual int64_t state_bytes() const = 0;
+    virtual void settle_state() = 0;
     virtual void read_state(size_t offset, size_t bytes, void* host) = 0;
     virtual void write_state(size_t offset, size_t bytes, const void* host) = 0;
     virtual void set_steps_done(int n) = 0;
@@ -130,6 +144,7 @@ struct ShotMem {
     void* arena = nullptr;  // 256-byte aligned; nullptr: the shot allocates its own
     size_t bytes = 0;       // usable bytes at arena
     bool inplace = false;   // one field set: no fused, double-buffered or overlapped schedule
+    bool one_set = false;   // one field set unless a measured or given launch shape asks for two
     int* host_flag = nullptr;  // pinned host int for the instability-flag readback
                                // (nullptr: the shot allocates one when first asked)
 };
@@ -150,12 +165,16 @@ void set_device_limit(int64_t bytes);  // <= 0: no limit
 // device address of the allocation-free entry point's static buffer on `device`
 // (ELA3D_NOALLOC_BYTES long; looked up once per device)
 void* noalloc_scratch(int device);
-Tuning choose_tuning(const ShotPlan& p);
+// launch shape of a new shot: the cached one (measured or given), else by rule; one_set: only
+// schedules that update in place are taken by rule
+Tuning choose_tuning(const ShotPlan& p, bool one_set = false);
 bool cached_tuning(const ela3d_config& c, Tuning& out);
 void store_tuning(const ela3d_config& c, const Tuning& t, double ms);
 // launch shapes of the absorbing-layer boxes (slab) and the interior box
 void geometry(const ShotPlan& p, const Tuning& t, LaunchGeom& slab, LaunchGeom& interior);
 // whether the fused schedule can run this plan with this tile (empty: yes)
 std::string fused_unsupported(const ShotPlan& p, int tile);
+// whether the whole-grid fused schedule can run this plan in this shape (empty: yes)
+std::string march_unsupported(const ShotPlan& p, const Tuning& t);
 
 }  // namespace ela3d

@@ -9,7 +9,8 @@
 // segment), all on a scratch shot of the same grid (source amplitude 0, so the
 // traffic is identical and nothing is perturbed).  The winner is cached keyed by
 // (nx, ny, nz, storage, npoints_pml); shots created with block = 0 and
-// zseg = 0 take the cached shape.
+// zseg = 0 take the cached shape.  Then come overlapped and merged launches, and the two
+// fused schedules (interior, whole grid).
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -54,7 +55,9 @@ bool cached_tuning(const ela3d_config& c, Tuning& out)
 void store_tuning(const ela3d_config& c, const Tuning& t, double ms)
 {
     std::lock_guard<std::mutex> g(tune_mutex());
-    tune_cache()[key_of(c)] = std::make_pair(t, ms);
+    Tuning u = t;
+    u.rule = 0;
+    tune_cache()[key_of(c)] = std::make_pair(u, ms);
 }
 
 }  // namespace ela3d
@@ -80,9 +83,21 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
         ela3d::ShotPlan plan = ela3d::make_plan(c);
         int n = 0;
         if (hipGetDeviceCount(&n) != hipSuccess || n <= c.device) throw Error{ELA3D_E_NODEVICE, "no HIP device"};
-        // a second field set lets the scratch shot also try the fused schedule
+        // a second field set lets the scratch shot also try the fused schedules
         const bool fusable = ela3d::fused_unsupported(plan, 1024).empty() || ela3d::fused_unsupported(plan, 512).empty();
-        std::unique_ptr<ela3d::Shot> shot = ela3d::make_shot(plan, cp, cs, rho, nullptr, fusable);
+        Tuning whole;
+        whole.fused = 2;
+        whole.dbuf = 1;
+        whole.tile = 256;
+        bool marchable = ela3d::march_unsupported(plan, whole).empty();
+        std::unique_ptr<ela3d::Shot> shot;
+        try {
+            shot = ela3d::make_shot(plan, cp, cs, rho, nullptr, fusable || marchable);
+        } catch (const Error& e) {
+            if (e.code != ELA3D_E_OOM || fusable) throw;
+            marchable = false;  // one set fits
+            shot = ela3d::make_shot(plan, cp, cs, rho, nullptr, false);
+        }
         static const int blocks[] = {64, 128, 256};
         static const int zsi[] = {1, 2, 4, 8, 16, 32};  // 1: more workgroups for small grids
         static const int zss[] = {1, 2, 4, 8};
@@ -237,8 +252,9 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
         if (wall3[1] < 0.97 * wall3[pick]) pick = 1;
         best = cand[pick];
         double best_wall = wall3[pick];
-        if (fusable) {  // fused interior step: tile x z segment; the fastest of them
-                        // replaces the two-pass pick if it is at least 1 % faster
+        if (fusable || marchable) {  // fused interior step: tile x z segment; whole-grid fused step:
+                                     // workgroup x z segment; the fastest of them replaces the
+                                     // two-pass pick if it is at least 1 % faster
             static const int tiles[] = {512, 768, 1024};
             static const int fzs[] = {4, 8, 12, 16, 24, 32};
             std::vector<std::pair<double, Tuning>> fc;
@@ -257,6 +273,23 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
                     fc.emplace_back(w, t);
                 }
             }
+            static const int mtiles[] = {256, 512, 1024};
+            static const int mzs2[] = {1, 2, 3, 4, 6, 8};
+            for (int tl : mtiles)
+                for (int z : mzs2) {
+                    Tuning t = best;
+                    t.overlap = 0;
+                    t.merged = 0;
+                    t.fused = 2;
+                    t.dbuf = 1;
+                    t.tile = tl;
+                    t.zseg_interior = z;
+                    t.strips = 4;
+                    if (!marchable || !ela3d::march_unsupported(plan, t).empty()) continue;
+                    const double w = wall_of(t);
+                    if (verbose) std::fprintf(stderr, "[tune] whole-grid workgroup %4d zseg %2d: %.4f ms\n", tl, z, w);
+                    fc.emplace_back(w, t);
+                }
             // the three fastest again, three rounds in turn with the two-pass pick,
             // each kept at its best round: their differences (under 1 %) are below
             // one short timing's noise
@@ -271,7 +304,8 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
             double fwall = 1e300;
             for (const auto& c : fc) {
                 if (verbose)
-                    std::fprintf(stderr, "[tune] fused finalist tile %4d zseg %2d: %.4f ms\n", c.second.tile,
+                    std::fprintf(stderr, "[tune] fused finalist (%s) tile %4d zseg %2d: %.4f ms\n",
+                                 c.second.fused == 2 ? "whole grid" : "interior", c.second.tile,
                                  c.second.zseg_interior, c.first);
                 if (c.first < fwall) {
                     fwall = c.first;
@@ -334,7 +368,7 @@ int ela3d_tuning_set(const ela3d_config* cfg, const ela3d_tuning* t)
     u.overlap = t->overlap ? 1 : 0;
     u.merged = t->merged ? 1 : 0;
     u.dbuf = t->dbuf ? 1 : 0;
-    u.fused = t->fused ? 1 : 0;
+    u.fused = t->fused == 2 ? 2 : t->fused ? 1 : 0;
     u.tile = t->tile > 0 ? t->tile : 1024;
     if (t->strips < 0 || t->strips > 64) return ELA3D_E_INVALID;
     u.strips = t->strips;

@@ -144,7 +144,7 @@ typedef struct ela3d_info {
     int32_t overlap;               /* absorbing-layer launches concurrent with the interior ones */
     int32_t merged;                /* one mixed launch per pass */
     int32_t dbuf;                  /* two field sets (double buffered) */
-    int32_t fused, tile;           /* fused interior schedule and its tile */
+    int32_t fused, tile;           /* fused schedule (1: interior, 2: whole grid) and its tile */
     int32_t strips;                /* fused: xy strips of its workgroup order in effect (0: up to 8) */
 } ela3d_info;
 
@@ -326,8 +326,10 @@ typedef struct ela3d_tuning {
     int32_t merged;       /* 1: one mixed launch per pass over every box (interior shape) */
     int32_t dbuf;         /* 1: two field sets; each step reads one and writes the other
                            * (FP32 and FP64 storage; FP16 storage always updates in place) */
-    int32_t fused;        /* 1: one fused stress+velocity launch over the interior box (needs dbuf) */
-    int32_t tile;         /* fused: interior cells per workgroup (multiple of 64, <= 1024) */
+    int32_t fused;        /* 1: one fused stress+velocity launch over the interior box (needs dbuf);
+                             2: one over the whole grid (needs dbuf) */
+    int32_t tile;         /* fused: interior cells per workgroup (multiple of 64, <= 1024); with 2,
+                             threads per workgroup: a wave per row of cells and one more */
     int32_t strips;       /* fused: xy strips the workgroup order walks, each through every z
                            * segment before the next (0 = the default: 4 for tiles of up to 768
                            * threads and at least 32 tiles per plane, else up to 8 strips of at
