@@ -202,8 +202,8 @@ __device__ __forceinline__ R quot(R dt, R r)
         return dt_quot(dt, r);
 }
 
-// a + b: with FP32 and FP64 never contracted with a product (see sum_r); FP16 storage
-// has one schedule only, and the compiler may
+// The updates' sums and products: written out with FP32 and FP64 (see sum_r); FP16 storage
+// has one schedule only, and the compiler contracts them
 template <typename T, typename R>
 __device__ __forceinline__ R sum(R a, R b)
 {
@@ -211,6 +211,26 @@ __device__ __forceinline__ R sum(R a, R b)
         return a + b;
     else
         return sum_r(a, b);
+}
+// a * b + c
+template <typename T, typename R>
+__device__ __forceinline__ R mad(R a, R b, R c)
+{
+    if constexpr (std::is_same<T, half_t>::value)
+        return a * b + c;
+    else
+        return fma_r(a, b, c);
+}
+template <typename T, typename R>
+__device__ __forceinline__ R cpml(R psi_old, R a, R b, R Kinv, R& d)
+{
+    if constexpr (std::is_same<T, half_t>::value) {
+        const R psi = b * psi_old + a * d;
+        d = d * Kinv + psi;
+        return psi;
+    } else {
+        return recur(psi_old, a, b, Kinv, d);
+    }
 }
 
 // acc + d, where d = diff * inv is the derivative along y or z, `layer` saying whether that
@@ -422,23 +442,27 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
         {
             onN[e] = L.act[e] && (i <= nx - 2) && (j >= 1) && (k >= 1 || surface);
             const R vp = P.cp_c[e];
-            const R lambda = Q.rho_c[e] * fma_r(vp, vp, (R)-2 * Q.cs_c[e] * Q.cs_c[e]);
+            R lambda;
+            if constexpr (std::is_same<T, half_t>::value)
+                lambda = Q.rho_c[e] * (vp * vp - (R)2 * Q.cs_c[e] * Q.cs_c[e]);
+            else
+                lambda = Q.rho_c[e] * fma_r(vp, vp, (R)-2 * Q.cs_c[e] * Q.cs_c[e]);
             const R l2m = Q.rho_c[e] * vp * vp;
             const R DT_l2m = dt * l2m, DT_l = dt * lambda;
             R dvx_dx = (P.vxE[e] - vx_c) * idx;
             R dvy_dy = (vy_c - P.vyS[e]) * idy;
             R dvz_dz = (P.vz_c[e] - Q.vz_m[e]) * idz;
             if (cx >= 0) {
-                const R m = recur(P.mx[0][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], dvx_dx);
+                const R m = cpml<T>(P.mx[0][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], dvx_dx);
                 if (onN[e]) stm(mout(A, 0), omx, m, S, 9);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = recur(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], dvy_dy);
+                    const R m = cpml<T>(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], dvy_dy);
                     if (onN[e]) stm(mout(A, 1), omy, m, S, 10);
                 }
                 if (Z.cz >= 0) {
-                    const R m = recur(P.mz[0][e], Z.az, Z.bz, Z.Kz, dvz_dz);
+                    const R m = cpml<T>(P.mz[0][e], Z.az, Z.bz, Z.Kz, dvz_dz);
                     if (onN[e]) stm(mout(A, 2), omz, m, S, 11);
                 }
             }
@@ -447,9 +471,16 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
                 // rate follows from lambda (exx + eyy) + (lambda + 2 mu) ezz = 0
                 dvz_dz = -(lambda / l2m) * sum<T>(dvx_dx, dvy_dy);
             }
-            nsxx[e] = sum<T>(fma_r(DT_l2m, dvx_dx, DT_l * sum<T>(dvy_dy, dvz_dz)), P.sxx[e]);
-            nsyy[e] = sum<T>(fma_r(DT_l2m, dvy_dy, DT_l * sum<T>(dvx_dx, dvz_dz)), P.syy[e]);
-            nszz[e] = surface ? P.szz[e] : sum<T>(fma_r(DT_l2m, dvz_dz, DT_l * sum<T>(dvx_dx, dvy_dy)), P.szz[e]);
+            if constexpr (std::is_same<T, half_t>::value) {
+                nsxx[e] = DT_l2m * dvx_dx + DT_l * (dvy_dy + dvz_dz) + P.sxx[e];
+                nsyy[e] = DT_l * (dvx_dx + dvz_dz) + DT_l2m * dvy_dy + P.syy[e];
+                nszz[e] = surface ? P.szz[e] : DT_l * (dvx_dx + dvy_dy) + DT_l2m * dvz_dz + P.szz[e];
+            } else {
+                nsxx[e] = sum_r(fma_r(DT_l2m, dvx_dx, DT_l * sum_r(dvy_dy, dvz_dz)), P.sxx[e]);
+                nsyy[e] = sum_r(fma_r(DT_l2m, dvy_dy, DT_l * sum_r(dvx_dx, dvz_dz)), P.syy[e]);
+                nszz[e] = surface ? P.szz[e]
+                                  : sum_r(fma_r(DT_l2m, dvz_dz, DT_l * sum_r(dvx_dx, dvy_dy)), P.szz[e]);
+            }
         }
         // sigma_xy: i in [1,nx-1], j in [0,ny-2]; mu averaged over (i-1,j),(i,j+1) (CPU:415-442)
         {
@@ -461,14 +492,14 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
             const R ey = P.vxN[e] - vx_c;
             R dvx_dy = ey * idy;
             if (cx >= 0) {
-                const R m = recur(P.mx[1][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvy_dx);
+                const R m = cpml<T>(P.mx[1][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvy_dx);
                 if (onXY[e]) stm(mout(A, 3), omx, m, S, 12);
             }
             if (MODE == kSlab && cy >= 0) {
-                const R m = recur(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvx_dy);
+                const R m = cpml<T>(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvx_dy);
                 if (onXY[e]) stm(mout(A, 4), omy, m, S, 13);
             }
-            nsxy[e] = fma_r(DT_mu, add_axis<T, MODE>(dvy_dx, ey, idy, dvx_dy, cy >= 0), P.sxy[e]);
+            nsxy[e] = mad<T>(DT_mu, add_axis<T, MODE>(dvy_dx, ey, idy, dvx_dy, cy >= 0), P.sxy[e]);
         }
         // sigma_xz: i in [1,nx-1]; mu averaged over (i-1,k),(i,k+1) (CPU:444-470)
         {
@@ -480,14 +511,14 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
             const R ez = P.vx_u[e] - vx_c;
             R dvx_dz = ez * idz;
             if (cx >= 0) {
-                const R m = recur(P.mx[2][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvz_dx);
+                const R m = cpml<T>(P.mx[2][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], dvz_dx);
                 if (onXZ[e]) stm(mout(A, 5), omx, m, S, 14);
             }
             if (MODE == kSlab && Z.cz >= 0) {
-                const R m = recur(P.mz[1][e], Z.azh, Z.bzh, Z.Kzh, dvx_dz);
+                const R m = cpml<T>(P.mz[1][e], Z.azh, Z.bzh, Z.Kzh, dvx_dz);
                 if (onXZ[e]) stm(mout(A, 6), omz, m, S, 15);
             }
-            nsxz[e] = fma_r(DT_mu, add_axis<T, MODE>(dvz_dx, ez, idz, dvx_dz, Z.cz >= 0), P.sxz[e]);
+            nsxz[e] = mad<T>(DT_mu, add_axis<T, MODE>(dvz_dx, ez, idz, dvx_dz, Z.cz >= 0), P.sxz[e]);
         }
         // sigma_yz: j in [0,ny-2]; mu averaged over (j+1,k),(j,k+1) (CPU:472-497)
         {
@@ -500,15 +531,15 @@ __device__ __forceinline__ void stress_update(const StepArgs<T>& A, const Lane<V
             R dvy_dz = ez * idz;
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = recur(P.my[2][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvz_dy);
+                    const R m = cpml<T>(P.my[2][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], dvz_dy);
                     if (onYZ[e]) stm(mout(A, 7), omy, m, S, 16);
                 }
                 if (Z.cz >= 0) {
-                    const R m = recur(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, dvy_dz);
+                    const R m = cpml<T>(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, dvy_dz);
                     if (onYZ[e]) stm(mout(A, 8), omz, m, S, 17);
                 }
             }
-            nsyz[e] = fma_r(DT_mu, add_axis<T, MODE>(dvz_dy, ez, idz, dvy_dz, Z.cz >= 0), P.syz[e]);
+            nsyz[e] = mad<T>(DT_mu, add_axis<T, MODE>(dvz_dy, ez, idz, dvy_dz, Z.cz >= 0), P.syz[e]);
         }
     }
     if constexpr (Scales<T>::on) {  // the source cell's new normal stresses go to the side slot
@@ -702,21 +733,21 @@ __device__ __forceinline__ void velocity_update(const StepArgs<T>& A, const Lane
             const R e3 = P.sxz[e] - (surface ? -P.sxz[e] : Q.sxz_m[e]);
             R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = recur(P.mx[0][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], d1);
+                const R m = cpml<T>(P.mx[0][e], (R)LT.x[0][e], (R)LT.x[1][e], (R)LT.x[2][e], d1);
                 if (onx) stm(mout(A, 9), omx, m, S, 18);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = recur(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
+                    const R m = cpml<T>(P.my[0][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
                     if (onx) stm(mout(A, 10), omy, m, S, 19);
                 }
                 if (Z.cz >= 0) {
-                    const R m = recur(P.mz[0][e], Z.az, Z.bz, Z.Kz, d3);
+                    const R m = cpml<T>(P.mz[0][e], Z.az, Z.bz, Z.Kz, d3);
                     if (onx) stm(mout(A, 11), omz, m, S, 20);
                 }
             }
             if (onx)
-                nvx[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vx[e]);
+                nvx[e] = mad<T>(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vx[e]);
         }
         // vy: i in [0,nx-2], j in [0,ny-2], k in [1,nz-1] (CPU:531-558), plane 0 at a free surface
         const bool ony = L.act[e] && (i <= nx - 2) && (j <= ny - 2) && (k >= 1 || surface);
@@ -730,21 +761,21 @@ __device__ __forceinline__ void velocity_update(const StepArgs<T>& A, const Lane
             const R e3 = P.syz[e] - (surface ? -P.syz[e] : Q.syz_m[e]);
             R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = recur(P.mx[1][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
+                const R m = cpml<T>(P.mx[1][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
                 if (ony) stm(mout(A, 12), omx, m, S, 21);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = recur(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], d2);
+                    const R m = cpml<T>(P.my[1][e], (R)LT.y[3][e], (R)LT.y[4][e], (R)LT.y[5][e], d2);
                     if (ony) stm(mout(A, 13), omy, m, S, 22);
                 }
                 if (Z.cz >= 0) {
-                    const R m = recur(P.mz[1][e], Z.az, Z.bz, Z.Kz, d3);
+                    const R m = cpml<T>(P.mz[1][e], Z.az, Z.bz, Z.Kz, d3);
                     if (ony) stm(mout(A, 14), omz, m, S, 23);
                 }
             }
             if (ony)
-                nvy[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vy[e]);
+                nvy[e] = mad<T>(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vy[e]);
         }
         // vz: i in [0,nx-2], j in [1,ny-1], k in [0,nz-2] (CPU:562-590)
         const bool onz = L.act[e] && (i <= nx - 2) && (j >= 1) && (k <= nz - 2);
@@ -758,21 +789,21 @@ __device__ __forceinline__ void velocity_update(const StepArgs<T>& A, const Lane
             const R e3 = P.szz_u[e] - Q.szz_c[e];
             R d3 = e3 * idz;
             if (cx >= 0) {
-                const R m = recur(P.mx[2][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
+                const R m = cpml<T>(P.mx[2][e], (R)LT.x[3][e], (R)LT.x[4][e], (R)LT.x[5][e], d1);
                 if (onz) stm(mout(A, 15), omx, m, S, 24);
             }
             if (MODE == kSlab) {
                 if (cy >= 0) {
-                    const R m = recur(P.my[2][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
+                    const R m = cpml<T>(P.my[2][e], (R)LT.y[0][e], (R)LT.y[1][e], (R)LT.y[2][e], d2);
                     if (onz) stm(mout(A, 16), omy, m, S, 25);
                 }
                 if (Z.cz >= 0) {
-                    const R m = recur(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, d3);
+                    const R m = cpml<T>(P.mz[2][e], Z.azh, Z.bzh, Z.Kzh, d3);
                     if (onz) stm(mout(A, 17), omz, m, S, 26);
                 }
             }
             if (onz)
-                nvz[e] = fma_r(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vz[e]);
+                nvz[e] = mad<T>(DT_over_rho, add_axis<T, MODE>(add_axis<T, MODE>(d1, e2, idy, d2, cy >= 0), e3, idz, d3, Z.cz >= 0), P.vz[e]);
         }
         // rigid faces: the memory variables above are still advanced, then v = 0
         const bool f = face && L.act[e];
