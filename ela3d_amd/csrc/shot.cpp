@@ -115,7 +115,7 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
     const ela3d_config& c = p.cfg;
     if (c.block == 0 && c.zseg == 0 && cached_tuning(c, t)) return t;
     t.rule = 1;
-    t.block = c.block > 0 ? c.block : 256;
+    t.block = c.block > 0 ? c.block : 128;
     t.block_slab = t.block;
     t.vec = 1;
     t.vec_slab = 1;
@@ -124,14 +124,20 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
         t.zseg_slab = c.zseg;
         return t;
     }
-    // enough workgroups to fill 256 CUs several times over; short z-segments
-    // measured best on MI355X (more waves in flight beats longer register queues)
-    const int64_t nchunk = (int64_t(c.nx) * (p.ax[1].hi - p.ax[1].lo) + t.block * t.vec - 1) / (t.block * t.vec);
-    const int nzi = std::max(1, p.ax[2].hi - p.ax[2].lo);
-    int zs = 8;
-    while (zs > 2 && nchunk * ((nzi + zs - 1) / zs) < 8192) zs /= 2;
+    // Two passes: short z segments measured best (more waves in flight beat longer register
+    // queues), interior and layers alike, down to one plane where a grid has too few
+    // workgroups for 256 CUs.  FP32 and FP64: 2 planes from 8,192 workgroups on (us, 1 / 2
+    // planes: 64^3 32 / 35, 101^3 51 / 53, 201^3 266 / 262, 401x401x301 1341 / 1311; FP64 120^3
+    // 102 / 110, 192x200x188 436 / 427).  FP16 moves half the bytes and its kernels are bound by
+    // instruction issue, to which a segment's start adds: 2 planes from 2,000 workgroups on, 4
+    // from 4,000 (64^3 1 / 2 planes 41 / 43, 101^3 2 / 4 61 / 67, 144^3 98 / 91, 401x401x301
+    // 934 / 868).
+    const bool half = c.storage == ELA3D_STORAGE_FP16;
+    const int64_t chunks = (int64_t(c.nx) * c.ny + t.block - 1) / t.block;
+    int zs = half ? 4 : 2;
+    while (zs > 1 && chunks * ((c.nz + zs - 1) / zs) < (half ? 1000 : 4096) * zs) zs /= 2;
     t.zseg_interior = zs;
-    t.zseg_slab = 4;
+    t.zseg_slab = zs;
     if (!one_set && c.block == 0) march_by_rule(p, t);
     return t;
 }
