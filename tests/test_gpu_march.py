@@ -138,3 +138,24 @@ def test_march_by_default(gpu, tmp_path, storage, dims, compat, fs):
             same(s)
     finally:
         set_device_limit(0)
+
+
+@pytest.mark.parametrize("storage,energy_every", [(STORAGE_FP32, 0), (STORAGE_FP32, 5), (STORAGE_FP64, 3), (1, 0)])
+def test_step_runs(gpu, storage, energy_every):
+    """Steps replayed in runs of every length and phase, with eager steps and synchronizations
+    between the replays, leave what eager launches leave: fields, samples and energies."""
+    cfg = small_cfg(nx=34, ny=21, nz=18, npml=4, nstep=150, storage=storage, src_kind=SRC_EXPLOSIVE,
+                    energy_every=energy_every)
+    model = hetero_model(cfg, seed=8)
+    with Shot(cfg.replace(use_graph=False), *model) as s:
+        s.run()
+        ref = [s.seismograms(), s.energy(), s.source_trace()] + fields(s)
+    with Shot(cfg, *model) as s:
+        for n in (1, 2, 2, 3, 16, 17, 17, 31, 2, 5, 5, 33):
+            s.step(n)
+            if n != 2:
+                s.sync()
+            s.profile(1) if n == 3 else None
+        s.run()
+        got = [s.seismograms(), s.energy(), s.source_trace()] + fields(s)
+    assert all(np.array_equal(x, y) for x, y in zip(ref, got))
