@@ -4,6 +4,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <atomic>
+#include <functional>
+#include <limits>
+#include <thread>
+#include <sched.h>
 
 namespace ela3d {
 
@@ -353,14 +358,70 @@ ShotPlan make_slab_plan(const ela3d_config& cfg, int k0, int k1, std::vector<int
     return P;
 }
 
-void check_model(int64_t cells, const float* cp, const float* cs, const float* rho)
+void parallel_ranges(int64_t n, int64_t grain, const std::function<void(int64_t, int64_t)>& fn)
 {
-    for (int64_t q = 0; q < cells; ++q) {
-        if (!(std::isfinite(cp[q]) && std::isfinite(cs[q]) && std::isfinite(rho[q])) || !(cs[q] > 0.f) ||
-            !(rho[q] > 0.f) || !(cp[q] > cs[q]))
-            throw Error{ELA3D_E_INVALID,
-                        "model cell " + std::to_string(q) + " invalid (need finite cp > cs > 0, rho > 0)"};
+    cpu_set_t set;
+    int cpus = 1;
+    if (sched_getaffinity(0, sizeof(set), &set) == 0) cpus = CPU_COUNT(&set);
+    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(std::min(8, cpus), n / grain));
+    std::vector<std::thread> pool;
+    int64_t next = n / parts;  // the caller runs the first range, and those no thread could be made for
+    try {
+        pool.reserve(size_t(parts));
+        for (int64_t q = 1; q < parts; ++q) {
+            const int64_t e = n * (q + 1) / parts;
+            pool.emplace_back(fn, next, e);
+            next = e;
+        }
+    } catch (...) {
     }
+    fn(0, n / parts);
+    if (next < n) fn(next, n);
+    for (auto& t : pool) t.join();
+}
+
+// Cells [b, e): the first invalid one, or e.  Blocks are tested without a branch per cell (the
+// compiler vectorizes them); cs is finite where it lies between 0 and a finite cp.
+static int64_t first_invalid(const float* cp, const float* cs, const float* rho, int64_t b, int64_t e)
+{
+    const float most = std::numeric_limits<float>::max();
+    for (int64_t q0 = b; q0 < e; q0 += 4096) {
+        const int64_t q1 = std::min(e, q0 + 4096);
+        int bad = 0;
+        for (int64_t q = q0; q < q1; ++q)
+            bad |= int(!(cp[q] <= most)) | int(!(cs[q] > 0.f)) | int(!(cp[q] > cs[q])) | int(!(rho[q] > 0.f)) |
+                   int(!(rho[q] <= most));
+        if (!bad) continue;
+        for (int64_t q = q0; q < q1; ++q)
+            if (!(cp[q] <= most) || !(cs[q] > 0.f) || !(cp[q] > cs[q]) || !(rho[q] > 0.f) || !(rho[q] <= most))
+                return q;
+    }
+    return e;
+}
+
+// One pass over the model, in ranges of half a million cells or more on up to 8 threads: a
+// loop with a branch per cell and condition took 1.4 ms at 101^3, a quarter of what creating
+// that shot took, and the server's copy 60 ms at 256^3, most of it first touches of its pages.
+void check_model(int64_t cells, const float* cp, const float* cs, const float* rho, float* copy)
+{
+    std::atomic<int64_t> bad{cells};
+    parallel_ranges(cells, int64_t(1) << 19, [&](int64_t b, int64_t e) {
+        const int64_t q = first_invalid(cp, cs, rho, b, e);
+        if (q < e) {
+            int64_t seen = bad.load();
+            while (q < seen && !bad.compare_exchange_weak(seen, q)) {
+            }
+        }
+        if (copy) {
+            const size_t n = size_t(e - b) * sizeof(float);
+            std::memcpy(copy + b, cp + b, n);
+            std::memcpy(copy + cells + b, cs + b, n);
+            std::memcpy(copy + 2 * cells + b, rho + b, n);
+        }
+    });
+    if (bad < cells)
+        throw Error{ELA3D_E_INVALID, "model cell " + std::to_string(bad.load()) +
+                                         " invalid (need finite cp > cs > 0, rho > 0)"};
 }
 
 int64_t device_bytes_estimate(const ela3d_config& c, const ShotPlan* plan, bool one_set)

@@ -1,6 +1,7 @@
 // core.hpp -- host-side shot description shared by the runtime, the server and the CLI.
 #pragma once
 
+#include <functional>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -91,8 +92,12 @@ PmlAxis make_axis(const ela3d_config& cfg, int axis);
 double wavelet_value(const ela3d_config& cfg, double t0, int it);
 // Device bytes a shot of this config holds (used by admission control).
 int64_t device_bytes_estimate(const ela3d_config& cfg, const ShotPlan* plan, bool one_set = false);
-// Throws ELA3D_E_INVALID unless every cell has finite cp > cs > 0 and rho > 0.
-void check_model(int64_t cells, const float* cp, const float* cs, const float* rho);
+// Throws ELA3D_E_INVALID unless every cell has finite cp > cs > 0 and rho > 0.  copy: 3 * cells
+// floats that receive cp, cs and rho, one after the other (nullptr: none).
+void check_model(int64_t cells, const float* cp, const float* cs, const float* rho, float* copy = nullptr);
+// fn(begin, end) over ranges that cover [0, n), each on a thread of its own and at least `grain`
+// long (a shorter n: one call here).  fn must not throw.
+void parallel_ranges(int64_t n, int64_t grain, const std::function<void(int64_t, int64_t)>& fn);
 // exact size of the single device allocation a shot of this plan makes
 int64_t shot_device_bytes(const ShotPlan& p, bool one_set = false);
 

@@ -154,6 +154,8 @@ constexpr int kMaxBatch = 64;  // shots in one batch launch
 void launch_copy(const float4* src, float4* dst, long n4, int variant, hipStream_t s);
 // zero `bytes` bytes at p (p 16-byte aligned) with a kernel on stream s
 void launch_zero(void* p, size_t bytes, hipStream_t s);
+// nz planes of n floats each, packed, to planes of `stride` floats
+void launch_planes(const float* src, float* dst, int n, int64_t stride, int nz, hipStream_t s);
 // Halo of a z interface: nf planes, each the first n elements at fields[q],
 // copied to (pack) or from (unpack) the contiguous buffer buf[nf][n].
 template <typename T>

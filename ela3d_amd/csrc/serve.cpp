@@ -120,7 +120,7 @@ struct Request {
     uint64_t ticket = 0;
     ela3d_config cfg{};
     std::vector<int32_t> rec;
-    std::vector<float> cp, cs, rho;
+    std::unique_ptr<float[]> model;  // cp, cs, rho, one after the other
     int64_t bytes = 0;           // device bytes charged to the budget
     bool one_set = false;        // steps in place unless its launch shape was measured or given
     std::atomic<int> state{ELA3D_SHOT_QUEUED};
@@ -216,14 +216,11 @@ public:
     uint64_t submit(const ela3d_config& cfg, const float* cp, const float* cs, const float* rho)
     {
         ShotPlan plan = make_plan(cfg);  // validates; throws Error
-        check_model(plan.cells, cp, cs, rho);
         auto r = std::unique_ptr<Request>(new Request);
         r->cfg = plan.cfg;
         r->rec = plan.rec;
-        const size_t n = size_t(plan.cells);
-        r->cp.assign(cp, cp + n);
-        r->cs.assign(cs, cs + n);
-        r->rho.assign(rho, rho + n);
+        r->model.reset(new float[3 * size_t(plan.cells)]);
+        check_model(plan.cells, cp, cs, rho, r->model.get());
         // Shots for the batch launches update in place, and so does one whose second field set
         // would not fit the budget.
         r->one_set = batchable(plan) || device_bytes_estimate(plan.cfg, &plan) > opts_.hbm_budget_bytes;
@@ -407,7 +404,9 @@ private:
             mem.bytes = need;
             mem.host_flag = sl.flag;
             mem.one_set = r->one_set;
-            r->shot = make_shot(std::move(plan), r->cp.data(), r->cs.data(), r->rho.data(), sl.stream, false, mem);
+            const float* cp = r->model.get();
+            const size_t cells = size_t(plan.cells);
+            r->shot = make_shot(std::move(plan), cp, cp + cells, cp + 2 * cells, sl.stream, false, mem);
             const int64_t actual = r->shot->device_bytes();
             {
                 std::lock_guard<std::mutex> g(mu_);
@@ -426,9 +425,7 @@ private:
                     ++batched_;
                 }
             }
-            std::vector<float>().swap(r->cp);  // the model now lives on the device
-            std::vector<float>().swap(r->cs);
-            std::vector<float>().swap(r->rho);
+            r->model.reset();  // the model now lives on the device
         } catch (const Error& e) {
             r->status = e.code;
             r->shot.reset();

@@ -763,10 +763,12 @@ public:
         const ela3d_config& c = plan_.cfg;
         const size_t cells = size_t(plan_.cells);
         if (field < 9) {
-            std::vector<T> h(cells);
-            copy_planes(h.data(), d_f_[cur()][field], sizeof(T), hipMemcpyDeviceToHost);
+            std::vector<T> h(size_t(nxyp_) * c.nz);
+            HIP_CHECK(hipMemcpy(h.data(), d_f_[cur()][field], h.size() * sizeof(T), hipMemcpyDeviceToHost));
             const double inv = 1.0 / current_scale(field);
-            for (size_t q = 0; q < cells; ++q) out[q] = double(h[q]) * inv;
+            each_plane([&](size_t to, size_t from, size_t n) {
+                for (size_t q = 0; q < n; ++q) out[to + q] = double(h[from + q]) * inv;
+            });
             if (side_mode() && field >= 3 && field <= 5) {  // the source cell lives in the side slot
                 float v = 0.f;
                 HIP_CHECK(hipMemcpy(&v, d_side_ + (field - 3), sizeof(float), hipMemcpyDeviceToHost));
@@ -790,20 +792,22 @@ public:
         HIP_CHECK(hipStreamSynchronize(stream_));
         const size_t cells = size_t(plan_.cells);
         if (field < 9) {
-            std::vector<T> h(cells);
+            std::vector<T> h(size_t(nxyp_) * plan_.cfg.nz, T(0));
             const bool side = side_mode() && field >= 3 && field <= 5;
             const size_t sc_cell = side ? src_cell() : cells;  // kept out of the FP16 array and its scale
             double mx = 0.0;
             for (size_t q = 0; q < cells; ++q)
                 if (q != sc_cell) mx = std::max(mx, std::fabs(in[q]));
             const double sc = host_scale(field, mx);
-            for (size_t q = 0; q < cells; ++q) h[q] = q == sc_cell ? T(0) : T(in[q] * sc);
+            each_plane([&](size_t from, size_t to, size_t n) {
+                for (size_t q = 0; q < n; ++q) h[to + q] = from + q == sc_cell ? T(0) : T(in[from + q] * sc);
+            });
             if (side) {
                 const float v = float(in[sc_cell]);
                 HIP_CHECK(hipMemcpy(d_side_ + (field - 3), &v, sizeof(float), hipMemcpyHostToDevice));
             }
             for (int b = 0; b < (dbuf_ ? 2 : 1); ++b)  // both sets: cells a step never writes keep it
-                copy_planes(d_f_[b][field], h.data(), sizeof(T), hipMemcpyHostToDevice);
+                HIP_CHECK(hipMemcpy(d_f_[b][field], h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
             return;
         }
         const int m = field - 9, axis = kMemAxis[m];
@@ -1109,20 +1113,32 @@ private:
         HIP_CHECK(hipMemcpy(d_scl_, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice));
     }
 
-    // host x-fastest nx*ny*nz  <->  device planes of stride nxyp_
-    void copy_planes(void* dst, const void* src, size_t elem, hipMemcpyKind kind)
+    // x-fastest nx*ny*nz host arrays and device planes of stride nxyp_: linear copies, the
+    // padding skipped on the host (fields) or spread on the device (the model)
+    template <typename F>
+    void each_plane(F fn) const
     {
-        const ela3d_config& c = plan_.cfg;
-        const size_t row = size_t(c.nx) * c.ny * elem, dev = size_t(nxyp_) * elem;
-        const bool to_dev = kind == hipMemcpyHostToDevice;
-        HIP_CHECK(hipMemcpy2D(dst, to_dev ? dev : row, src, to_dev ? row : dev, row, size_t(c.nz), kind));
+        const size_t n = size_t(plan_.cfg.nx) * plan_.cfg.ny;
+        for (size_t k = 0; k < size_t(plan_.cfg.nz); ++k) fn(k * n, k * size_t(nxyp_), n);
     }
 
     void upload(const float* cp, const float* cs, const float* rho)
     {
         const ela3d_config& c = plan_.cfg;
         const float* src[3] = {cp, cs, rho};
-        for (int q = 0; q < 3; ++q) copy_planes(d_model_[q], src[q], sizeof(float), hipMemcpyHostToDevice);
+        const size_t cells = size_t(plan_.cells), bytes = cells * sizeof(float);
+        if (nxyp_ == int64_t(c.nx) * c.ny) {
+            for (int q = 0; q < 3; ++q) HIP_CHECK(hipMemcpy(d_model_[q], src[q], bytes, hipMemcpyHostToDevice));
+        } else {  // by way of the fields (the arena's start; 18 bytes a cell or more), cleared again
+            float* packed = static_cast<float*>(arena_);
+            for (int q = 0; q < 3; ++q) {
+                float* at = packed + size_t(q) * cells;
+                HIP_CHECK(hipMemcpy(at, src[q], bytes, hipMemcpyHostToDevice));
+                launch_planes(at, d_model_[q], c.nx * c.ny, nxyp_, c.nz, stream_);
+            }
+            launch_zero(arena_, 3 * bytes, stream_);
+            HIP_CHECK(hipGetLastError());
+        }
         for (int a = 0; a < 3; ++a) {
             const PmlAxis& A = plan_.ax[a];
             std::vector<double> t(6 * size_t(A.n));
