@@ -209,7 +209,8 @@ k_fused(const StepArgs<T> A)
     const Box B = A.box[0];
     const int nx = A.nx, ny = A.ny, LR = A.ldsreg;
     int chunk, zs;
-    tile_of(B, xcd_block(blockIdx.x, gridDim.x), chunk, zs);
+    const int blk = turned(blockIdx.x, gridDim.x, A.back);
+    tile_of(B, xcd_block(blk, gridDim.x), chunk, zs);
     const int own_full = fused_own(A.tile, nx);
     const int q0 = B.p0 + chunk * own_full;
     const int n = min(own_full, B.p1 - q0);
@@ -434,8 +435,8 @@ k_fused(const StepArgs<T> A)
                 a += red[0][w];
                 bsum += red[1][w];
             }
-            A.epart[2 * blockIdx.x] = a;
-            A.epart[2 * blockIdx.x + 1] = bsum;
+            A.epart[2 * blk] = a;
+            A.epart[2 * blk + 1] = bsum;
         }
     }
 }

@@ -19,6 +19,15 @@ __host__ __device__ inline int xcd_block(int b, int n)
     return x * q + (x < r ? x : r) + l;
 }
 
+// Block b of n with each XCD's blocks taken in reverse: xcd_block of the result walks an XCD's
+// logical range backwards.  Also a bijection.
+__host__ __device__ inline int turned(int b, int n, int back)
+{
+    if (!back) return b;
+    const int x = b % 8, l = b / 8;
+    return (n / 8 + (x < n % 8 ? 1 : 0) - 1 - l) * 8 + x;
+}
+
 // Box of logical block lb in a launch over nbox boxes (blk0 ascending).
 __host__ __device__ inline Box pick_box(const Box* bx, int nbox, int lb)
 {

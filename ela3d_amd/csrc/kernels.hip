@@ -905,7 +905,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& A, int lb)
 template <typename T, int MODE, int V>
 __global__ void __launch_bounds__(256) k_stress(const StepArgs<T> A)
 {
-    stress_block<T, MODE, V>(A, xcd_block(blockIdx.x, gridDim.x));
+    stress_block<T, MODE, V>(A, xcd_block(turned(blockIdx.x, gridDim.x, A.back), gridDim.x));
 }
 
 // shot of logical block lb in a batch launch (blk0 ascending, nshot small)
@@ -967,7 +967,8 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& A, int lb, int
 template <typename T, int MODE, bool ENERGY, int V>
 __global__ void __launch_bounds__(256) k_velocity(const StepArgs<T> A)
 {
-    velocity_block<T, MODE, ENERGY, V>(A, xcd_block(blockIdx.x, gridDim.x), blockIdx.x);
+    const int blk = turned(blockIdx.x, gridDim.x, A.back);
+    velocity_block<T, MODE, ENERGY, V>(A, xcd_block(blk, gridDim.x), blk);
 }
 
 template <typename T, int V>

@@ -86,6 +86,7 @@ struct StepArgs {
     int tile;                // kFused: threads per workgroup = region cells (own cells + 2 halo rows)
     int ldsreg;              // kFused: cells of one LDS stress plane (= tile)
     int rows;                // kMarch: rows a workgroup owns
+    int back;                // 1: workgroups walk the grid backwards (see turned)
     int xch, xw;             // kMarch: x chunks, and the columns each owns
 };
 

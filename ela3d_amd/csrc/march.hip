@@ -659,7 +659,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) 
     const Box B = A.box[0];
     const int nx = A.nx, ny = A.ny;
     int chunk, zs;
-    tile_of(B, xcd_block(blockIdx.x, gridDim.x), chunk, zs);
+    const int blk = turned(blockIdx.x, gridDim.x, A.back);
+    tile_of(B, xcd_block(blk, gridDim.x), chunk, zs);
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const MarchTile t = march_tile(nx, ny, A.rows, A.xch, A.xw, chunk);
     March<T> M{A};
@@ -745,8 +746,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) 
                 a += red[0][q];
                 b += red[1][q];
             }
-            A.epart[2 * blockIdx.x] = a;
-            A.epart[2 * blockIdx.x + 1] = b;
+            A.epart[2 * blk] = a;
+            A.epart[2 * blk + 1] = b;
         }
     }
 }

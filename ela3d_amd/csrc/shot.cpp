@@ -406,6 +406,12 @@ private:
         set_args();
     }
 
+    // bytes of the arrays a step reads and writes
+    int64_t state_moved() const
+    {
+        return int64_t(arena_layout(plan_, int(sizeof(T)), 0, dbuf_ ? kSetAppended : kOneSet).total);
+    }
+
     // sets, overlap and geometry of tune_
     void set_shape(bool asked)
     {
@@ -1238,6 +1244,13 @@ private:
         a.tile = g.tile;
         a.ldsreg = g.tile;
         a.rows = g.rows;
+        // Every other pass over the grid goes backwards where what one step moves is more than the
+        // last-level cache holds but not more than four times that: a pass then starts with what
+        // the one before it touched last, still cached (one launch a step: 144^3 105 -> 99 us,
+        // 160^3 134 -> 125, 201^3 244 -> 232; two passes: 201^3 256 -> 244, FP16 256^3 343 -> 336).
+        // Larger grids and cached ones gain nothing and lose up to 1 %.
+        const bool turn = state_moved() > kInfinityCache && state_moved() <= 4 * kInfinityCache;
+        a.back = !turn ? 0 : tune_.fused ? par : pass;
         a.xch = g.xch;
         a.xw = g.xw;
         return a;

@@ -69,6 +69,18 @@ int main(int argc, char** argv)
                               (long long)w[2] * ny * nx - cut};
     std::vector<unsigned char> cells(size_t(nx) * ny * nz, 0), ms[3];
     for (int q = 0; q < 3; ++q) ms[q].assign(size_t(mem[q] + cut), 0);
+    // walked backwards, an XCD's blocks are the same ones in reverse
+    for (int n = 1; n <= G.nblocks; n = n < 40 || n == G.nblocks ? n + 1 : G.nblocks) {
+        std::vector<unsigned char> seen(size_t(n), 0);
+        for (int b = 0; b < n; ++b) {
+            const int x = b % 8, len = n / 8 + (x < n % 8 ? 1 : 0), t = turned(b, n, 1);
+            if (turned(b, n, 0) != b || t < 0 || t >= n || seen[size_t(t)]++) {
+                ++g_bad;
+                break;
+            }
+            if (xcd_block(t, n) - xcd_block(x, n) != len - 1 - b / 8) ++g_bad;
+        }
+    }
     for (int b = 0; b < G.nblocks; ++b) {
         int chunk, zs, kb, ke;
         tile_of(G.box[0], xcd_block(b, G.nblocks), chunk, zs);
