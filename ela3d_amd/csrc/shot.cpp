@@ -66,12 +66,11 @@ constexpr int64_t kInfinityCache = int64_t(256) << 20;
 // It reads and writes every array once per step (two passes: about 1.6 times the bytes) but
 // keeps two field sets and, with few columns per wave, idles lanes.  Measured, us per step,
 // two passes against one launch:
-//  * launch-bound and small grids: 33^3 30 -> 19, 64^3 33 -> 24, 101^3 51 -> 43;
-//  * beyond the 256 MiB cache: 201^3 261 -> 253, 256^3 490 -> 446, 401x401x301 1311 -> 1200,
-//    480x500x360 2252 -> 2030, FP64 192x200x188 424 -> 379;
-//  * where one set stays in the cache and two do not, two passes stay ahead: 144^3 93 / 119,
-//    160^3 115 / 145, 170^3 156 / 171, FP64 120^3 101 / 126 (at 180^3, one set 1.2 times the
-//    cache, both take the same);
+//  * launch-bound and small grids: 33^3 19 / 12, 64^3 23 / 18, 101^3 43 / 40, 128^3 67 / 62;
+//  * beyond the 256 MiB cache: 180^3 181 / 166, 201^3 244 / 229, 300x110x150 151 / 140,
+//    401x401x301 1305 / 1182, 480x500x360 2250 / 1953, FP64 144^3 187 / 168, 192x200x188 423 / 353;
+//  * where one set stays in the cache and two do not, two passes stay ahead: 200x120x120 83 / 98,
+//    144^3 88 / 99, 160^3 109 / 125, FP64 110^3 78 / 81, 120^3 101 / 122;
 //  * with more workgroups than fit at once and fewer than 0.6 of a wave's lanes on columns, the
 //    lanes decide: 65x800x640 (0.51) 1013 / 1091, 72x800x640 (0.56) 1095 / 1122, 80x800x640
 //    (0.63) 1195 / 1145, 130x600x640 (0.68) 1425 / 1403.
@@ -84,19 +83,33 @@ static bool march_by_rule(const ShotPlan& p, Tuning& t)
     Tuning m = t;
     m.fused = 2;
     m.dbuf = 1;
-    // Workgroup: short ones (3 rows and the halo wave) balance best over the grids measured; FP64
-    // has registers for half as many waves and more halo arithmetic per row, so 7 rows.
-    m.tile = dbl ? 512 : 256;
-    m.strips = 4;
     // z segment: the shortest whose workgroups are all on the chip at once (24 waves per compute
-    // unit, FP64 16); at most 6 planes, where the planes reloaded at a segment's ends cost less
-    // than the imbalance of longer ones (401x401x301: 4 / 6 / 8 planes 1195 / 1203 / 1242 us,
-    // 256^3: 457 / 446 / 458).
+    // unit, FP64 16), up to 6 planes; where none is, 4 (FP64 5): the planes reloaded at a
+    // segment's ends cost less than the disorder of longer ones (4 / 6 / 8 planes, us: 201^3
+    // 231 / 238 / 248, 401x401x301 1185 / 1226 / 1259, 480x500x360 1964 / 2022 / 2102, FP64 144^3
+    // 168 / 171 / 181, 192x200x188 362 / 354 / 353).
+    // Workgroup: 7 rows and the halo wave.  FP32 grids that are on the chip at once, but not with
+    // one plane, balance better in workgroups of 3 rows (7 / 3 rows, us: 72^3 27 / 26, 90^3
+    // 34 / 32, 101^3 41 / 38; with one plane 57^3 16 / 17, 64^3 18 / 19; FP64 81x61x75 32 / 41).
+    m.strips = 4;
     int xch = 0;
-    const int xw = march_chunk_width(c.nx, xch), rows = m.tile / 64 - 1;
-    const int64_t tiles = int64_t((c.ny + rows - 1) / rows) * xch, fit = int64_t(256) * (dbl ? 16 : 24) * 64 / m.tile;
-    int z = 1;
-    while (z < 6 && tiles * ((c.nz + z - 1) / z) > fit) ++z;
+    march_chunk_width(c.nx, xch);
+    int64_t tiles = 0, fit = 0;
+    auto shortest = [&](int tile) {
+        const int rows = tile / 64 - 1;
+        m.tile = tile;
+        tiles = int64_t((c.ny + rows - 1) / rows) * xch;
+        fit = int64_t(256) * (dbl ? 16 : 24) * 64 / tile;
+        int z = 1;
+        while (z <= 6 && tiles * ((c.nz + z - 1) / z) > fit) ++z;
+        return z;
+    };
+    int z = shortest(512);
+    if (!dbl && z > 1) {
+        z = shortest(256);
+        if (z > 6) z = shortest(512);
+    }
+    if (z > 6) z = dbl ? 5 : 4;
     m.zseg_interior = z;
     if (!march_unsupported(p, m).empty()) return false;
     if (tiles * ((c.nz + z - 1) / z) > fit && c.nx * 10 < xch * 64 * 6) return false;
@@ -104,7 +117,7 @@ static bool march_by_rule(const ShotPlan& p, Tuning& t)
     const int64_t one = int64_t(arena_layout(p, elem, 0, kOneSet).total);
     const int64_t two = int64_t(arena_layout(p, elem, 0, kSetAppended).total);
     if (two > (int64_t(16) << 30)) return false;
-    if (two > kInfinityCache && one < kInfinityCache / 4 * 5) return false;
+    if (two > kInfinityCache && one <= kInfinityCache) return false;
     t = m;
     return true;
 }
@@ -125,17 +138,17 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
         return t;
     }
     // Two passes: short z segments measured best (more waves in flight beat longer register
-    // queues), interior and layers alike, down to one plane where a grid has too few
-    // workgroups for 256 CUs.  FP32 and FP64: 2 planes from 8,192 workgroups on (us, 1 / 2
-    // planes: 64^3 32 / 35, 101^3 51 / 53, 201^3 266 / 262, 401x401x301 1341 / 1311; FP64 120^3
-    // 102 / 110, 192x200x188 436 / 427).  FP16 moves half the bytes and its kernels are bound by
-    // instruction issue, to which a segment's start adds: 2 planes from 2,000 workgroups on, 4
-    // from 4,000 (64^3 1 / 2 planes 41 / 43, 101^3 2 / 4 61 / 67, 144^3 98 / 91, 401x401x301
-    // 934 / 868).
+    // queues), interior and layers alike, down to one plane where a grid has few workgroups
+    // for 256 CUs or lies in the last-level cache.  FP32 and FP64: 2 planes from 20,000 workgroups
+    // on (us, 1 / 2 planes: 64^3 32 / 35, 101^3 51 / 53, 144^3 91 / 94, 160^3 113 / 115, 201^3
+    // 247 / 244, 401x401x301 1338 / 1305; FP64 120^3 102 / 110, 192x200x188 436 / 427).  FP16 moves
+    // half the bytes and its kernels are bound by instruction issue, to which a segment's start
+    // adds: 2 planes from 2,000 workgroups on, 4 from 4,000 (64^3 1 / 2 planes 41 / 43, 101^3
+    // 2 / 4 61 / 67, 144^3 98 / 91, 401x401x301 934 / 868).
     const bool half = c.storage == ELA3D_STORAGE_FP16;
     const int64_t chunks = (int64_t(c.nx) * c.ny + t.block - 1) / t.block;
     int zs = half ? 4 : 2;
-    while (zs > 1 && chunks * ((c.nz + zs - 1) / zs) < (half ? 1000 : 4096) * zs) zs /= 2;
+    while (zs > 1 && chunks * ((c.nz + zs - 1) / zs) < (half ? 1000 : 10000) * zs) zs /= 2;
     t.zseg_interior = zs;
     t.zseg_slab = zs;
     if (!one_set && c.block == 0) march_by_rule(p, t);
