@@ -108,7 +108,8 @@ struct TailArgs {
     int nwavelet;
     int src_kind, src, nx, nxy;  // nxy: plane stride of the device layout
     double sin_t, cos_t, dt;
-    int* step;               // steps completed (device counter)
+    const int* step;         // steps completed (device counter)
+    int* step_out;           // receives the new count (in place the same word)
     int* flag;               // set to 1 when a sample or the energy is not finite
     float* scl;              // FP16 storage scale table (see kScaleTable)
     float* side;             // FP16 with a stress source: the source cell's normal stresses (see StepArgs)
@@ -116,6 +117,14 @@ struct TailArgs {
     int rescale_every;       // FP16 storage: re-choose every scale each N steps
     double* srctrace;        // [nstep+1][3] sigma_xx, sigma_yy, sigma_zz at the source after injection
     int nsrctrace;           // rows of srctrace
+    // Whole-grid fused step: a launch also records the step before it, whose set it reads, if
+    // `record` is set; g: vx, vy, vz, sigma_xx, sigma_yy, sigma_zz of that set; pre_in, pre_out:
+    // the source cell's velocities before the injection of the recorded step and of this one
+    const T* g[6];
+    const double* pre_in;
+    double* pre_out;
+    int is, js, ks;          // source cell
+    int record;
 };
 
 template <typename T>
@@ -137,7 +146,10 @@ size_t fused_lds_bytes(int nx, int tile);
 // fused step over the whole grid, absorbing layers included (march.hip); needs
 // double-buffered fields.  A workgroup has a wave per own row and two halo waves.
 template <typename T>
-void launch_march(const StepArgs<T>& a, bool energy, hipStream_t s);
+void launch_march(const StepArgs<T>& a, const TailArgs<T>& tail, bool energy, hipStream_t s);
+// records the last step of a run of them (`block` threads, as the step's workgroups)
+template <typename T>
+void launch_record(const TailArgs<T>& a, int block, hipStream_t s);
 template <typename T>
 void launch_tail(const TailArgs<T>& a, hipStream_t s);
 // A batch of shots stepped together (each a merged launch over all its boxes,

@@ -27,8 +27,8 @@
 // Updates follow the reference CPU loops (seismicCPML_3d_isotropic_simpelmodel.cpp):
 // normal stress CPU:377-413, sigma_xy CPU:415-442, sigma_xz/yz CPU:444-499,
 // vx/vy CPU:501-560, vz CPU:562-590.
-#include "device_util.hpp"
 #include "geom.hpp"
+#include "tail_util.hpp"
 
 // Every multiply-add is written out: a cell's result is then the same bits whichever wave
 // computes it (own or halo row, general or plain code).
@@ -37,6 +37,7 @@
 namespace ela3d {
 namespace {
 
+constexpr int kLead = 8;  // workgroups before the grid's own, one per die
 // roles of a wave
 constexpr int kOwn = 0, kLow = 1, kHigh = 2;
 // phases of a plane: below the segment (sigma_xz and sigma_yz only), in it, above it (sigma_zz only)
@@ -652,15 +653,26 @@ __device__ __forceinline__ void march_halo(const March<T>& ML, const March<T>& M
 }
 
 template <typename T, bool ENERGY, int NT, int WPE>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) k_march(const StepArgs<T> A)
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) k_march(const StepArgs<T> A, const TailArgs<T> E)
 {
     typedef typename Arith<T>::R R;
     extern __shared__ double march_smem[];
     const Box B = A.box[0];
     const int nx = A.nx, ny = A.ny;
     int chunk, zs;
-    const int blk = turned(blockIdx.x, gridDim.x, A.back);
-    tile_of(B, xcd_block(blk, gridDim.x), chunk, zs);
+    // A leading workgroup records the step before this one meanwhile (a tail kernel after every
+    // step took 4 us: 64^3 18.0 -> 15.3 us a step, 101^3 37.8 -> 35.1).  Seven idle ones beside it
+    // keep the others on the dies they would be on: moved by one die each, the two that march
+    // through one strip no longer neighbour each other (401x401x301: 1176 -> 1207 us).
+    if (blockIdx.x < kLead) {
+        if (blockIdx.x > 0) return;
+        const int done = *E.step;
+        if (E.record) record_step(E, done, march_smem);
+        if (threadIdx.x == 0) *E.step_out = done + 1;
+        return;
+    }
+    const int nb = int(gridDim.x) - kLead, blk = turned(int(blockIdx.x) - kLead, nb, A.back);
+    tile_of(B, xcd_block(blk, nb), chunk, zs);
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const MarchTile t = march_tile(nx, ny, A.rows, A.xch, A.xw, chunk);
     March<T> M{A};
@@ -750,22 +762,44 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) 
             A.epart[2 * blk + 1] = b;
         }
     }
+    // the source, once its workgroup has stored every cell
+    if (E.is >= t.x0 && E.is < t.x1 && E.js >= t.j0 && E.js < t.j0 + t.n && E.ks >= M.kb && E.ks < M.ke) {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int q = 0; q < 3; ++q) E.pre_out[q] = (double)E.f[q][E.src];
+            inject_source(E, *E.step + 1, static_cast<float*>(nullptr));
+        }
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kMarchThreads) k_record(const TailArgs<T> E)
+{
+    __shared__ double red[2 * kMarchThreads / 64];
+    record_step(E, *E.step, red);
 }
 
 }  // namespace
 
 template <typename T>
-void launch_march(const StepArgs<T>& a, bool energy, hipStream_t s)
+void launch_march(const StepArgs<T>& a, const TailArgs<T>& tail, bool energy, hipStream_t s)
 {
     constexpr int NT = kMarchThreads / (sizeof(T) / 4), WPE = sizeof(T) == 4 ? 6 : 4;
     const size_t lds = march_lds_bytes(int(sizeof(T)), a.rows, a.box[0].zseg);
     if (a.nblocks <= 0 || a.block != 64 * (a.rows + 1) || a.block > NT || lds > kMarchLds) return;  // refused on the host first
     if (energy)
-        hipLaunchKernelGGL((k_march<T, true, NT, WPE>), dim3(a.nblocks), dim3(a.block), lds, s, a);
+        hipLaunchKernelGGL((k_march<T, true, NT, WPE>), dim3(a.nblocks + kLead), dim3(a.block), lds, s, a, tail);
     else
-        hipLaunchKernelGGL((k_march<T, false, NT, WPE>), dim3(a.nblocks), dim3(a.block), lds, s, a);
+        hipLaunchKernelGGL((k_march<T, false, NT, WPE>), dim3(a.nblocks + kLead), dim3(a.block), lds, s, a, tail);
 }
-template void launch_march<float>(const StepArgs<float>&, bool, hipStream_t);
-template void launch_march<double>(const StepArgs<double>&, bool, hipStream_t);
+template <typename T>
+void launch_record(const TailArgs<T>& a, int block, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_record<T>), dim3(1), dim3(block), 0, s, a);
+}
+template void launch_march<float>(const StepArgs<float>&, const TailArgs<float>&, bool, hipStream_t);
+template void launch_march<double>(const StepArgs<double>&, const TailArgs<double>&, bool, hipStream_t);
+template void launch_record<float>(const TailArgs<float>&, int, hipStream_t);
+template void launch_record<double>(const TailArgs<double>&, int, hipStream_t);
 
 }  // namespace ela3d

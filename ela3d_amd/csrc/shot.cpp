@@ -264,6 +264,10 @@ std::string fused_unsupported(const ShotPlan& p, int tile)
     return "the grid has no interior box";
 }
 
+// control words of a shot: step count of set 0, instability flag, step count of set 1, and from
+// byte 16 the source cell's velocities before the injection, [set][3]
+constexpr size_t kCtlBytes = 16 + 6 * sizeof(double);
+
 static int epart_capacity(const ela3d_config& c)
 {
     return int((plane_stride(c.nx, c.ny) / 64 + kMaxBox + 1) * int64_t(c.nz) + 8);
@@ -282,7 +286,8 @@ std::string march_unsupported(const ShotPlan& p, const Tuning& t)
     if (march_lds_bytes(elem, t.tile / 64 - 1, std::max(1, t.zseg_interior)) > kMarchLds) return "the row buffers do not fit the LDS";
     LaunchGeom slab, all;
     geometry(p, t, slab, all);
-    if (all.nblocks > epart_capacity(c)) return "too many workgroups for the energy partials";
+    // (a set of partials each for the step in progress and the one being recorded)
+    if (2 * int64_t(all.nblocks) > epart_capacity(c)) return "too many workgroups for the energy partials";
     return "";
 }
 
@@ -333,7 +338,7 @@ ArenaLayout arena_layout(const ShotPlan& p, int elem, int nepart, Sets sets)
     L.epart_cap = epart_capacity(c);
     L.epart = off; off += al(size_t(std::max(L.epart_cap, nepart)) * 2 * sizeof(double));
     L.epart2 = off; off += al(size_t(kEpartBlocks) * 2 * sizeof(double));
-    L.ctl = off; off += al(2 * sizeof(int));
+    L.ctl = off; off += al(kCtlBytes);
     L.scl = off; off += al(kScaleTable * sizeof(float));
     L.slot = off; off += al(size_t(kMaxSlots) * 27 * sizeof(unsigned));
     L.srctrace = off; off += al((size_t(c.nstep) + 1) * 3 * sizeof(double));
@@ -504,6 +509,7 @@ public:
             const size_t n = mem_elems(plan_, kMemAxis[q]) * sizeof(T);
             if (n) HIP_CHECK(hipMemcpyAsync(b + L.m[q], b + L.m2[q], n, hipMemcpyDeviceToDevice, stream_));
         }
+        HIP_CHECK(hipMemcpyAsync(step_word(0), step_word(1), sizeof(int), hipMemcpyDeviceToDevice, stream_));
         par_ = 0;
     }
 
@@ -605,7 +611,7 @@ public:
         unsigned energy = 0;  // bit s: step s of the run sums the energy
         for (int s = 0; s < n; ++s) energy |= unsigned(energy_step(host_step_ + 1 + s)) << s;
         if (!plan_.cfg.use_graph) {
-            for (int s = 0; s < n; ++s) launch_step(energy >> s & 1u, nullptr, dbuf_ ? (par + s) & 1 : 0);
+            launch_run(n, energy, par);
         } else if (StepGraph& g = graph_of(n, energy, par); g.exec) {
             HIP_CHECK(hipGraphLaunch(g.exec, stream_));
         } else {
@@ -663,7 +669,7 @@ public:
         for (int s = 0; s < n; ++s) {
             const int done = host_step_;
             const int it = done + 1;
-            HIP_CHECK(hipMemcpyAsync(d_step_, &done, sizeof(int), hipMemcpyHostToDevice, stream_));
+            HIP_CHECK(hipMemcpyAsync(step_word(cur()), &done, sizeof(int), hipMemcpyHostToDevice, stream_));
             HIP_CHECK(hipStreamSynchronize(stream_));
             launch_step(energy_step(it), nullptr, cur());
             HIP_CHECK(hipGetLastError());
@@ -773,6 +779,9 @@ public:
     {
         host_step_ = n;
         par_ = sets_ == kTwoSets ? n & 1 : 0;  // an appended set's state is restored to the first
+        if (dbuf_)
+            for (int set = 0; set < 2; ++set)
+                HIP_CHECK(hipMemcpy(step_word(set), &n, sizeof(int), hipMemcpyHostToDevice));
     }
 
     void snapshot(int field, double* out) override
@@ -1076,6 +1085,7 @@ private:
         d_epart2_ = reinterpret_cast<double*>(b + L.epart2);
         d_step_ = reinterpret_cast<int*>(b + o_ctl);
         d_flag_ = d_step_ + 1;
+        d_presrc_ = reinterpret_cast<double*>(d_step_ + 4);
         d_scl_ = reinterpret_cast<float*>(b + o_scl);
         d_maxslot_ = reinterpret_cast<unsigned*>(b + o_slot);
         d_srctrace_ = reinterpret_cast<double*>(b + o_src);
@@ -1247,7 +1257,7 @@ private:
         a.maxslot = d_maxslot_;
         a.side = side_mode() ? d_side_ : nullptr;
         a.sidx = unsigned(guard_) + unsigned(src_offset());
-        a.epart = epart;
+        a.epart = g.mode == kMarch ? epart + 2 * size_t(out) * nepart_ : epart;
         for (int q = 0; q < g.nbox; ++q) a.box[q] = g.box[q];
         a.nbox = g.nbox;
         a.nblocks = g.nblocks;
@@ -1293,7 +1303,8 @@ private:
         const ela3d_config& c = plan_.cfg;
         TailArgs<T> a;
         std::memset(&a, 0, sizeof(a));
-        for (int q = 0; q < 9; ++q) a.f[q] = d_f_[dbuf_ ? 1 - par : par][q];
+        const int out = dbuf_ ? 1 - par : par;
+        for (int q = 0; q < 9; ++q) a.f[q] = d_f_[out][q];
         a.cp = d_model_[0];
         a.rho = d_model_[2];
         a.rec = d_rec_;
@@ -1317,7 +1328,8 @@ private:
         a.sin_t = std::sin(th);
         a.cos_t = std::cos(th);
         a.dt = c.dt;
-        a.step = d_step_;
+        a.step = step_word(par);
+        a.step_out = step_word(out);
         a.flag = d_flag_;
         a.scl = d_scl_;
         a.maxslot = d_maxslot_;
@@ -1325,7 +1337,25 @@ private:
         a.rescale_every = std::max(1, c.fp16_rescale_every);
         a.srctrace = d_srctrace_;
         a.nsrctrace = c.nstep + 1;
+        if (tune_.fused == 2) {
+            record_from(a, par);
+            a.pre_out = d_presrc_ + 3 * out;
+        }
         return a;
+    }
+
+    // whole-grid fused step: the set to record
+    void record_from(TailArgs<T>& a, int set) const
+    {
+        const ela3d_config& c = plan_.cfg;
+        for (int q = 0; q < 6; ++q) a.g[q] = d_f_[set][q];
+        a.step = step_word(set);
+        a.epart = d_epart_ + 2 * size_t(set) * nepart_;
+        a.nepart = nepart_;
+        a.pre_in = d_presrc_ + 3 * set;
+        a.is = c.isrc;
+        a.js = c.jsrc;
+        a.ks = c.ksrc;
     }
 
     // One time step: stress pass -> velocity pass -> tail (receivers, energy, source).
@@ -1336,7 +1366,9 @@ private:
     // stream in sequence.  With ev != nullptr, events ev[2q], ev[2q+1] bracket
     // launch q (stress layers, stress interior, velocity layers, velocity
     // interior, tail) on the stream it runs on.
-    void launch_step(bool energy, hipEvent_t* ev, int par)
+    // record: the whole-grid fused step also records the step before it (receivers, energy,
+    // source trace); last: and nothing records this one later
+    void launch_step(bool energy, hipEvent_t* ev, int par, bool record = false, bool last = true)
     {
         auto mark = [&](int q, hipStream_t s) {
             if (ev) HIP_CHECK(hipEventRecord(ev[q], s));
@@ -1346,12 +1378,17 @@ private:
             mark(2, stream_);
             if constexpr (std::is_same<T, half_t>::value)
                 throw Error{ELA3D_E_INVALID, "the fused schedule does not run FP16 storage"};
-            else
-                launch_march(args_[par][0][0], energy, stream_);
-            for (int q = 3; q < 9; ++q) mark(q, stream_);
-            if (energy) launch_epart(d_epart_, nepart_, d_epart2_, epart_blocks(), stream_);
-            launch_tail(tail_args(par), stream_);
-            mark(9, stream_);
+            else {
+                TailArgs<T> a = tail_args(par);
+                a.record = record ? 1 : 0;
+                launch_march(args_[par][0][0], a, energy, stream_);
+                for (int q = 3; q < 9; ++q) mark(q, stream_);
+                if (last) {
+                    record_from(a, 1 - par);
+                    launch_record(a, tune_.tile, stream_);
+                }
+                mark(9, stream_);
+            }
             return;
         }
         if (tune_.fused) {  // layers' stresses, the fused interior step, layers' velocities
@@ -1404,6 +1441,13 @@ private:
         mark(9, stream_);
     }
 
+    // n steps from set par, energy sums in those of the mask
+    void launch_run(int n, unsigned energy, int par)
+    {
+        for (int s = 0; s < n; ++s)
+            launch_step(energy >> s & 1u, nullptr, dbuf_ ? (par + s) & 1 : 0, s > 0, s == n - 1);
+    }
+
     // the run of graph_run as a graph; a capture that fails leaves the stream out of capture
     hipGraphExec_t capture(int n, unsigned energy, int par)
     {
@@ -1411,7 +1455,7 @@ private:
         hipGraphExec_t exec = nullptr;
         HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
         try {
-            for (int s = 0; s < n; ++s) launch_step(energy >> s & 1u, nullptr, dbuf_ ? (par + s) & 1 : 0);
+            launch_run(n, energy, par);
         } catch (...) {
             (void)hipStreamEndCapture(stream_, &graph);
             if (graph) (void)hipGraphDestroy(graph);
@@ -1463,6 +1507,9 @@ private:
     double* d_tab_[3] = {};
     double *d_wav_ = nullptr, *d_seis_ = nullptr, *d_energy_ = nullptr, *d_epart_ = nullptr;
     double* d_epart2_ = nullptr;  // first-level sums of the energy partials
+    double* d_presrc_ = nullptr;  // [set][3] source-cell velocities before the injection
+    // device count of the steps done, one word per set (a launch reads one and writes the other)
+    int* step_word(int set) const { return d_step_ + (set ? 2 : 0); }
     int *d_rec_ = nullptr, *d_step_ = nullptr, *d_flag_ = nullptr;
     int nepart_ = 0, epart_cap_ = 0;
     int64_t nxyp_ = 0, guard_ = 0;

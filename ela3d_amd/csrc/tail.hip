@@ -2,54 +2,9 @@
 // counter) and the stream-copy kernel used to calibrate the HBM ceiling.
 #include <algorithm>
 
-#include "device_util.hpp"
+#include "tail_util.hpp"
 
 namespace ela3d {
-
-// scale of the data written this step (FP16 storage; 1 otherwise)
-template <typename T>
-__device__ __forceinline__ float nsc(const TailArgs<T>& A, int q)
-{
-    if constexpr (std::is_same<T, half_t>::value) return A.scl[54 + q];
-    return 1.f;
-}
-template <typename T>
-__device__ __forceinline__ float nisc(const TailArgs<T>& A, int q)
-{
-    if constexpr (std::is_same<T, half_t>::value) return A.scl[81 + q];
-    return 1.f;
-}
-
-// source injection into field q at cell o, recording the magnitude written
-template <typename T>
-__device__ __forceinline__ void inject(const TailArgs<T>& A, int q, int o, typename Arith<T>::R v, float* inj)
-{
-    stf(A.f[q], o, v, nsc<T>(A, q));
-    inj[q] = fabsf((float)v);
-}
-
-// stress injection at the source cell: into the side slot where FP16 storage
-// keeps the source cell's normal stresses there (see StepArgs::side)
-template <typename T>
-__device__ __forceinline__ void inject_sigma(const TailArgs<T>& A, int q, int o, typename Arith<T>::R add, float* inj)
-{
-    if constexpr (std::is_same<T, half_t>::value) {
-        if (A.side) {
-            A.side[q - 3] = A.side[q - 3] + (float)add;
-            return;
-        }
-    }
-    inject(A, q, o, ldf(A.f[q], o, nisc<T>(A, q)) + add, inj);
-}
-
-template <typename T>
-__device__ __forceinline__ double sigma_at_source(const TailArgs<T>& A, int q, int o)
-{
-    if constexpr (std::is_same<T, half_t>::value) {
-        if (A.side) return (double)A.side[q - 3];
-    }
-    return (double)ldf(A.f[q], o, nisc<T>(A, q));
-}
 
 // ---------------------------------------------------------------------------
 // Per-step tail (one workgroup): receivers (before the source, as CPU:593-602
@@ -112,46 +67,7 @@ __device__ __forceinline__ void tail_body(const TailArgs<T>& A)
     }
     __syncthreads();
     if (tid == 0) {
-        if (it - 1 < A.nwavelet) {
-            const double st = A.wavelet[it - 1];
-            const int o = A.src;
-            const R DT = (R)A.dt;
-            const R l2m = (R)A.rho[o] * (R)A.cp[o] * (R)A.cp[o];
-            switch (A.src_kind) {
-            case 0: {  // CPU:620-622
-                const R fx = (R)(A.sin_t * st), fy = (R)(A.cos_t * st);
-                inject_sigma(A, 3, o, fx * DT * l2m, inj);
-                inject_sigma(A, 4, o, fx * DT * l2m, inj);
-                inject_sigma(A, 5, o, fy * DT * l2m, inj);
-                break;
-            }
-            case 1: {  // CPU:614-617
-                const R fx = (R)(A.sin_t * st), fy = (R)(A.cos_t * st);
-                const R rx = ((R)A.rho[o] + (R)A.rho[o - 1]) / (R)2;
-                const R ry = ((R)A.rho[o] + (R)A.rho[o + A.nx]) / (R)2;
-                inject(A, 0, o, ldf(A.f[0], o, nisc<T>(A, 0)) + fx * DT / rx, inj);
-                inject(A, 1, o, ldf(A.f[1], o, nisc<T>(A, 1)) + fy * DT / ry, inj);
-                break;
-            }
-            case 2: {
-                const R s = (R)st;
-                inject_sigma(A, 3, o, s * DT * l2m, inj);
-                inject_sigma(A, 4, o, s * DT * l2m, inj);
-                inject_sigma(A, 5, o, s * DT * l2m, inj);
-                break;
-            }
-            default: {  // ZC:451-453
-                const R s = (R)st;
-                const R rx = ((R)A.rho[o] + (R)A.rho[o - 1]) / (R)2;
-                const R ry = ((R)A.rho[o] + (R)A.rho[o + A.nx]) / (R)2;
-                const R rz = ((R)A.rho[o] + (R)A.rho[o + A.nxy]) / (R)2;
-                inject(A, 0, o, ldf(A.f[0], o, nisc<T>(A, 0)) + s * DT / rx, inj);
-                inject(A, 1, o, ldf(A.f[1], o, nisc<T>(A, 1)) + s * DT / ry, inj);
-                inject(A, 2, o, ldf(A.f[2], o, nisc<T>(A, 2)) + s * DT / rz, inj);
-                break;
-            }
-            }
-        }
+        inject_source(A, it, inj);
         // the velocities and normal stresses at the source cell after injection, all
         // loaded at once: the stresses are the source trace (UNI:463-465), and every
         // step, whatever the receivers and energy cadence, a non-finite one marks the
@@ -167,7 +83,7 @@ __device__ __forceinline__ void tail_body(const TailArgs<T>& A)
         }
         const bool fin = isfinite(sxx) && isfinite(syy) && isfinite(szz) && isfinite(vx) && isfinite(vy) && isfinite(vz);
         if (bad || !fin) *A.flag = 1;
-        *A.step = it;
+        *A.step_out = it;
     }
     if constexpr (std::is_same<T, half_t>::value) {
         // FP16 storage: the data now sits at the "next" scales; make them current

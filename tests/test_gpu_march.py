@@ -176,3 +176,40 @@ def test_turned_passes(gpu):
         for q, x in enumerate(a):
             assert np.array_equal(x, s.snapshot(q)), q
         assert np.array_equal(s.seismograms(), seis) and rel_l2(s.energy(), en) <= 1e-6
+
+
+@pytest.mark.parametrize("storage", [STORAGE_FP32, STORAGE_FP64])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+@pytest.mark.parametrize("cell", [(0.5, 0.5, 0.5), (0.1, 0.9, 0.2)])
+def test_recording(gpu, storage, kind, cell):
+    """What ends a step is recorded by the launch after it, or at a run's end by one of its own:
+    samples (a receiver on the source cell, more receivers than threads), energies, source trace
+    are those of the two-pass tail, whatever the runs; steps past the wavelet's end too."""
+    cfg = small_cfg(nx=67, ny=19, nz=17, npml=3, nstep=47, storage=storage, src_kind=kind, energy_every=3)
+    src = [int(f * n) for f, n in zip(cell, (67, 19, 17))]
+    rng = np.random.default_rng(1)
+    rec = np.vstack([[src], rng.integers(1, (66, 18, 16), size=(600, 3))]).astype(np.int32)
+    cfg = cfg.replace(isrc=src[0], jsrc=src[1], ksrc=src[2], receivers=rec, sample_every=2)
+    model = hetero_model(cfg, seed=12)
+    with Shot(cfg.replace(block=128, zseg=2), *model) as s:
+        s.run()
+        ref, seis, en, tr = fields(s), s.seismograms(), s.energy(), s.source_trace()
+    assert np.any(seis[:, 0])
+    for runs, graph in (((47,), True), ((1, 2, 16, 16, 12), True), ((5, 42), False)):
+        with Shot(cfg.replace(use_graph=graph), *model) as s:
+            assert s.info()["fused"] == 2
+            for n in runs:
+                s.step(n)
+            s.sync()
+            assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
+            assert np.array_equal(s.seismograms(), seis) and np.array_equal(s.source_trace(), tr)
+            assert rel_l2(s.energy(), en) <= (1e-6 if storage == STORAGE_FP32 else 1e-13)
+
+
+def test_recording_flags_a_blow_up(gpu):
+    cfg = small_cfg(nx=40, ny=20, nz=18, npml=3, nstep=600, src_kind=SRC_FORCE3)
+    cfg = cfg.replace(dt=4.0 * cfg.dt)
+    with Shot(cfg, *hetero_model(cfg, seed=1)) as s:
+        assert s.info()["fused"] == 2
+        with pytest.raises(Exception):
+            s.run()
