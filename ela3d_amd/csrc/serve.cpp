@@ -122,7 +122,7 @@ struct Request {
     std::vector<int32_t> rec;
     std::unique_ptr<float[]> model;  // cp, cs, rho, one after the other
     int64_t bytes = 0;           // device bytes charged to the budget
-    bool one_set = false;        // steps in place unless its launch shape was measured or given
+    bool one_set = false;        // placed without the whole-grid step's second field set
     std::atomic<int> state{ELA3D_SHOT_QUEUED};
     std::atomic<int> status{ELA3D_OK};
     double t_submit = 0, t_admit = 0, t_done = 0;
@@ -419,7 +419,7 @@ private:
             if (batching() && !opts_.plain_loop && r->shot->plan().cells <= int64_t(opts_.batch_cells) &&
                 int(batch_.members.size()) < kMaxBatch) {
                 BatchMember probe;
-                if (r->shot->batch_member(kBatchBlock, probe)) {
+                if (r->shot->batch_member(kBatchBlock, 1, probe)) {
                     r->batched = true;
                     batch_.members.push_back(r);
                     ++batched_;
@@ -531,9 +531,15 @@ private:
                 auto* ta = reinterpret_cast<TailArgs<float>*>(va + kMaxBatch);
                 auto* blk = reinterpret_cast<int*>(ta + kMaxBatch);
                 int nb = 0;
+                // planes per workgroup: by the workgroups of all members together, as for one
+                // shot (choose_tuning).  Six shots of 64^3 to 114^3, ten of 48^3 to 100^3, ms
+                // for 600 steps with 1 / 2 / 4 planes: 74 / 68 / 72, 72 / 68 / 73.
+                int64_t cells = 0;
+                for (Request* r : step) cells += r->shot->plan().cells;
+                const int zseg = cells / (2 * kBatchBlock) >= 8192 ? 2 : 1;
                 for (size_t q = 0; q < step.size(); ++q) {
                     BatchMember m;
-                    if (!step[q]->shot->batch_member(kBatchBlock, m)) throw Error{ELA3D_E_STATE, "shot left the batch"};
+                    if (!step[q]->shot->batch_member(kBatchBlock, zseg, m)) throw Error{ELA3D_E_STATE, "shot left the batch"};
                     sa[q] = m.stress;
                     va[q] = m.velocity;
                     ta[q] = m.tail;

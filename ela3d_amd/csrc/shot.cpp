@@ -126,8 +126,10 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
 {
     Tuning t;
     const ela3d_config& c = p.cfg;
-    if (c.block == 0 && c.zseg == 0 && cached_tuning(c, t)) return t;
-    t.rule = 1;
+    if (c.block == 0 && c.zseg == 0 && cached_tuning(c, t)) {
+        if (!(one_set && t.fused == 2)) return t;
+        t = Tuning();
+    }
     t.block = c.block > 0 ? c.block : 128;
     t.block_slab = t.block;
     t.vec = 1;
@@ -413,8 +415,8 @@ private:
         if (overlap_) make_aux();
         try {
             allocate();
-        } catch (const Error& e) {  // no room for the second set of a schedule taken by rule
-            if (e.code != ELA3D_E_OOM || !tune_.rule || !dbuf_ || dbuf) throw;
+        } catch (const Error& e) {  // no room for the second set of the whole-grid step
+            if (e.code != ELA3D_E_OOM || sets_ != kSetAppended) throw;
             tune_ = choose_tuning(plan_, true);
             set_shape(false);
             allocate();
@@ -475,7 +477,7 @@ public:
     void enqueue_phase(int phase) override
     {
         HIP_CHECK(hipSetDevice(device_));
-        if (tune_.rule && sets_ == kSetAppended && dbuf_) leave_second_set();
+        if (tune_.fused == 2 && sets_ == kSetAppended) leave_second_set();
         if (tune_.fused || dbuf_ || overlap_)
             throw Error{ELA3D_E_STATE, "stepping by phases needs the in-place two-pass schedule"};
         const int it = host_step_ + 1;
@@ -513,8 +515,7 @@ public:
         par_ = 0;
     }
 
-    // From a schedule with two sets that was taken by rule to two passes in place: for calls
-    // that only those serve.  The second set stays allocated, unused.
+    // From the whole-grid step to two passes in place, for calls that only those serve.  The second set stays allocated, unused.
     void leave_second_set()
     {
         to_first_set();
@@ -684,10 +685,11 @@ public:
         HIP_CHECK(hipStreamSynchronize(stream_));
     }
 
-    bool batch_member(int block, BatchMember& out) override
+    bool batch_member(int block, int zseg, BatchMember& out) override
     {
         if constexpr (!std::is_same<T, float>::value) {
             (void)block;
+            (void)zseg;
             (void)out;
             return false;
         } else {
@@ -695,6 +697,7 @@ public:
             Tuning t = tune_;
             t.block = block;
             t.vec = 1;
+            if (plan_.cfg.zseg == 0) t.zseg_interior = t.zseg_slab = zseg;
             t.merged = 1;
             t.fused = 0;
             t.overlap = 0;

@@ -50,7 +50,6 @@ struct Tuning {
     int tile = 1024;        // fused: interior cells of the flattened plane per workgroup (1);
                             //    threads per workgroup, a wave per own row and two more (2)
     int strips = 0;         // fused: xy strips of the tile order (0: the default of tile_of)
-    int rule = 0;           // 1: chosen by choose_tuning's rules, not measured or given
 };
 
 // Device layout of the 9 fields and the 3 model arrays: planes of plane_stride
@@ -91,10 +90,10 @@ public:
     // queue a copy of the instability flag into pinned host memory; after the
     // stream has passed that point, unstable_seen() reports it without a sync
     virtual void enqueue_flag_readback(hipStream_t on = nullptr) = 0;  // on: another stream
-    // Arguments of this shot as a member of a batch launch of `block` threads
-    // (one merged launch per pass over all its boxes); false if the shot cannot
+    // Arguments of this shot as a member of a batch launch of `block` threads, `zseg` planes
+    // per workgroup (one merged launch per pass over all its boxes); false if the shot cannot
     // be batched (not FP32, double-buffered or with energy sums).
-    virtual bool batch_member(int block, BatchMember& out) = 0;
+    virtual bool batch_member(int block, int zseg, BatchMember& out) = 0;
     virtual bool unstable_seen() const = 0;
     virtual void seismograms(double* out) = 0;      // nsamples*nrec*3
     virtual void energy(double* out) = 0;           // nenergy*2
@@ -144,7 +143,7 @@ struct ShotMem {
     void* arena = nullptr;  // 256-byte aligned; nullptr: the shot allocates its own
     size_t bytes = 0;       // usable bytes at arena
     bool inplace = false;   // one field set: no fused, double-buffered or overlapped schedule
-    bool one_set = false;   // one field set unless a measured or given launch shape asks for two
+    bool one_set = false;   // no whole-grid step, which needs a second field set
     int* host_flag = nullptr;  // pinned host int for the instability-flag readback
                                // (nullptr: the shot allocates one when first asked)
 };
@@ -165,8 +164,8 @@ void set_device_limit(int64_t bytes);  // <= 0: no limit
 // device address of the allocation-free entry point's static buffer on `device`
 // (ELA3D_NOALLOC_BYTES long; looked up once per device)
 void* noalloc_scratch(int device);
-// launch shape of a new shot: the cached one (measured or given), else by rule; one_set: only
-// schedules that update in place are taken by rule
+// launch shape of a new shot: the cached one (measured or given), else by rule; one_set: two
+// passes in place of the whole-grid step
 Tuning choose_tuning(const ShotPlan& p, bool one_set = false);
 bool cached_tuning(const ela3d_config& c, Tuning& out);
 void store_tuning(const ela3d_config& c, const Tuning& t, double ms);

@@ -55,9 +55,7 @@ bool cached_tuning(const ela3d_config& c, Tuning& out)
 void store_tuning(const ela3d_config& c, const Tuning& t, double ms)
 {
     std::lock_guard<std::mutex> g(tune_mutex());
-    Tuning u = t;
-    u.rule = 0;
-    tune_cache()[key_of(c)] = std::make_pair(u, ms);
+    tune_cache()[key_of(c)] = std::make_pair(t, ms);
 }
 
 }  // namespace ela3d

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import oracle
-from ela3d_amd import (COMPAT_REFERENCE, SRC_EXPLOSIVE, SRC_FORCE3, STORAGE_FP32, STORAGE_FP64, Shot, set_device_limit,
+from ela3d_amd import (COMPAT_REFERENCE, SRC_EXPLOSIVE, SRC_FORCE3, STORAGE_FP32, STORAGE_FP64, Server, Shot, set_device_limit,
                        set_tuning)
 from helpers import compare_state, hetero_model, max_rel, push_state, random_state, rel_l2, small_cfg
 from test_march_index import checker, run as address_check  # noqa: F401
@@ -213,3 +213,24 @@ def test_recording_flags_a_blow_up(gpu):
         assert s.info()["fused"] == 2
         with pytest.raises(Exception):
             s.run()
+
+
+def test_pinned_whole_grid_step_gives_way(gpu):
+    """A measured or given whole-grid shape steps by phases in place too, and a shot of that grid
+    that has to update in place (served in a batch, or without room for two sets) takes two passes."""
+    cfg = small_cfg(nx=52, ny=22, nz=20, npml=3, nstep=24, src_kind=SRC_EXPLOSIVE, energy_every=0)
+    model = hetero_model(cfg, seed=4)
+    set_tuning(cfg, block=128, zseg_interior=2, zseg_slab=2, fused=2, tile=320)
+    with Shot(cfg, *model) as s:
+        assert s.info()["fused"] == 2 and s.info()["tile"] == 320
+        s.step(3)
+        s.step_phase(0)
+        s.step_phase(1)
+        assert s.info()["fused"] == 0 and s.info()["steps_done"] == 4
+        s.run()
+        seis = s.seismograms()
+    with Server(max_active=3) as srv:
+        tickets = [srv.submit(cfg, *model) for _ in range(3)]
+        out = [srv.result(t) for t in tickets]
+        assert srv.stats()["batched"] == 3
+    assert all(np.array_equal(o[0], seis) for o in out)
