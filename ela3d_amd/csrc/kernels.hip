@@ -86,7 +86,9 @@ struct Scales {
     float r[27], w[27], mx[27];
     __device__ __forceinline__ void track(int q, float v)
     {
-        if constexpr (on) mx[q] = fmaxf(mx[q], fabsf(v));
+        // fmaxf(mx, fabsf(v)) in one instruction (the compiler adds a canonicalization of mx and a
+        // move); a NaN leaves mx as it is
+        if constexpr (on) asm("v_max_f32 %0, %0, |%1|" : "+v"(mx[q]) : "v"(v));
     }
 };
 
