@@ -532,7 +532,7 @@ def main():
             "workload": desc, "nx": cfg.nx, "ny": cfg.ny, "nz": cfg.nz,
             "cells": cfg.cells, "npoints_pml": cfg.npoints_pml, "nrec": cfg.nrec,
             "energy_every": cfg.energy_every,
-            "schedule": "fused interior step" if info["fused"] else "two-pass (stress, velocity)",
+            "schedule": ("two-pass (stress, velocity)", "fused interior step", "whole-grid fused step")[info["fused"]],
             "timing": (f"{K} steps: every {args.profile_every}-th eager with hipEvents around each launch "
                        "(roofline), the others hipGraph replays"),
             "alg_bytes_per_step": info["alg_bytes_per_step"],

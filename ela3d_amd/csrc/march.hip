@@ -12,17 +12,18 @@
 //    sets of row buffers, so one LDS barrier per plane orders everything;
 //  * z neighbours: registers, carried from plane to plane.
 // 24 (FP64 16) waves per compute unit with no spilled register are what hides the loads:
-// variants with two or four columns per lane (half the waves, misaligned vectors), with the
-// next plane's loads in flight across the barrier (10 to 20 registers spilled), and with
-// streaming loads or stores were 5 to 30 % slower at 401 x 401 x 301.  The halo rows share a
-// wave: alone they leave it idle for half a plane (101^3: 47 -> 41 us a step).
+// variants with two or four columns per lane (half the waves, misaligned vectors) and with
+// streaming loads or stores were 5 to 30 % slower at 401 x 401 x 301, the next plane's loads
+// issued before the barrier (73 registers for 67) 2 %, 32 waves (spills) 5 %.  The halo rows
+// share a wave: one each would be idle for half a plane (101^3: 47 -> 41 us a step).
 //
-// Time per step, FP32, against two passes of two launches: 33^3 30 -> 19 us, 101^3 51 -> 41,
-// 201^3 261 -> 248, 401x401x301 1311 -> 1180, 480x500x360 2252 -> 1990; FP64 81x61x75 47 -> 37,
-// 192x200x188 424 -> 375.  The small grids are bound by launches and latency.  The large ones
-// move 0.6 of the two passes' bytes (401x401x301: 5.4 GB, 1.15 times what one read and one write
-// of every array would be) at 4.6 TB/s, where a copy with as many streams reaches 5.6; what is
-// left is the latency of a plane's one load -> barrier -> store chain.
+// Time per step, FP32, two passes of two launches and a tail against this: 33^3 19 -> 10 us,
+// 64^3 23 -> 15, 101^3 43 -> 35, 201^3 244 -> 228, 401x401x301 1305 -> 1173, 480x500x360
+// 2250 -> 1950; FP64 81x61x75 39 -> 30, 192x200x188 423 -> 353.  The small grids are bound by a
+// chain of latencies: the tables, the plane below, each plane, the plane above.  The large
+// ones move 5.5 GB a step at 401x401x301 (two passes 6.4), 1.2 times one read and one write of
+// every array, at 4.7 TB/s, where a copy with as many streams reaches 5.6: a segment's ends are
+// read again, and rows beside a tile where workgroups have drifted apart.
 //
 // Updates follow the reference CPU loops (seismicCPML_3d_isotropic_simpelmodel.cpp):
 // normal stress CPU:377-413, sigma_xy CPU:415-442, sigma_xz/yz CPU:444-499,

@@ -66,9 +66,9 @@ constexpr int64_t kInfinityCache = int64_t(256) << 20;
 // It reads and writes every array once per step (two passes: about 1.6 times the bytes) but
 // keeps two field sets and, with few columns per wave, idles lanes.  Measured, us per step,
 // two passes against one launch:
-//  * launch-bound and small grids: 33^3 19 / 12, 64^3 23 / 18, 101^3 43 / 40, 128^3 67 / 62;
+//  * launch-bound and small grids: 33^3 19 / 10, 64^3 23 / 15, 101^3 43 / 35, 128^3 67 / 59;
 //  * beyond the 256 MiB cache: 180^3 181 / 166, 201^3 244 / 229, 300x110x150 151 / 140,
-//    401x401x301 1305 / 1182, 480x500x360 2250 / 1953, FP64 144^3 187 / 168, 192x200x188 423 / 353;
+//    401x401x301 1305 / 1173, 480x500x360 2250 / 1950, FP64 144^3 187 / 168, 192x200x188 423 / 353;
 //  * where one set stays in the cache and two do not, two passes stay ahead: 200x120x120 83 / 98,
 //    144^3 88 / 99, 160^3 109 / 125, FP64 110^3 78 / 81, 120^3 101 / 122;
 //  * with more workgroups than fit at once and fewer than 0.6 of a wave's lanes on columns, the

@@ -48,7 +48,7 @@ struct Tuning {
                             // 2: one fused launch over the whole grid (needs dbuf;
                             //    zseg_interior planes per workgroup)
     int tile = 1024;        // fused: interior cells of the flattened plane per workgroup (1);
-                            //    threads per workgroup, a wave per own row and two more (2)
+                            //    threads per workgroup, a wave per own row and one more (2)
     int strips = 0;         // fused: xy strips of the tile order (0: the default of tile_of)
 };
 
