@@ -358,6 +358,9 @@ private:
             for (size_t q = 0; q < active_.size(); ++q)
                 if (!active_[q]->batched) progressed |= advance(active_[q]);
             if (batching()) progressed |= advance_batch();
+            // Copies of models that are on the device by now: given back once the first steps are
+            // enqueued (200 MB take 10 ms, and the GPU would wait for them).
+            for (Request* r : admitted) r->model.reset();
             // retire finished shots
             for (size_t q = 0; q < active_.size();) {
                 Request* r = active_[q];
@@ -425,7 +428,6 @@ private:
                     ++batched_;
                 }
             }
-            r->model.reset();  // the model now lives on the device
         } catch (const Error& e) {
             r->status = e.code;
             r->shot.reset();
