@@ -116,7 +116,7 @@ typedef struct ela3d_config {
     int32_t dirichlet;      /* 1: vx=vy=vz=0 on the six faces after each velocity update */
     int32_t fp16_rescale_every; /* FP16 storage: re-choose scales every N steps (default 100) */
     int32_t device;         /* HIP device ordinal */
-    int32_t use_graph;      /* 1 (default): replay a hipGraph of one step */
+    int32_t use_graph;      /* 1 (default): replay hipGraphs of up to 16 steps */
     int32_t block;          /* threads per workgroup, 0 = autotuned */
     int32_t zseg;           /* z planes per workgroup, 0 = autotuned */
     int32_t free_surface;   /* 1: traction-free surface at the plane k = 0 (no z-min C-PML
@@ -274,7 +274,7 @@ typedef struct ela3d_server_opts {
     int64_t hbm_budget_bytes;  /* admission budget for shot device memory (default 200 GB) */
     int32_t max_active;        /* shots resident and stepping at once (default 16) */
     int32_t steps_per_round;   /* steps enqueued per shot between completion checks (default 50) */
-    int32_t use_graph;         /* replay a hipGraph per step (default 1) */
+    int32_t use_graph;         /* replay hipGraphs of steps (default 1) */
     int32_t plain_loop;        /* 1: reference-pattern one-shot-at-a-time loop */
     int32_t batch_cells;       /* FP32 shots of at most this many cells without energy sums
                                 * step together, one stress, one velocity and one tail launch
