@@ -122,14 +122,11 @@ static bool march_by_rule(const ShotPlan& p, Tuning& t)
     return true;
 }
 
-Tuning choose_tuning(const ShotPlan& p, bool one_set)
+// The two-pass schedule of a shape that was not measured.
+static Tuning two_pass_by_rule(const ShotPlan& p)
 {
     Tuning t;
     const ela3d_config& c = p.cfg;
-    if (c.block == 0 && c.zseg == 0 && cached_tuning(c, t)) {
-        if (!(one_set && t.fused == 2)) return t;
-        t = Tuning();
-    }
     t.block = c.block > 0 ? c.block : 128;
     t.block_slab = t.block;
     t.vec = 1;
@@ -139,7 +136,7 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
         t.zseg_slab = c.zseg;
         return t;
     }
-    // Two passes: short z segments measured best (more waves in flight beat longer register
+    // Short z segments measured best (more waves in flight beat longer register
     // queues), interior and layers alike, down to one plane where a grid has few workgroups
     // for 256 CUs or lies in the last-level cache.  FP32 and FP64: 2 planes from 20,000 workgroups
     // on (us, 1 / 2 planes: 64^3 32 / 35, 101^3 51 / 53, 144^3 91 / 94, 160^3 113 / 115, 201^3
@@ -153,7 +150,28 @@ Tuning choose_tuning(const ShotPlan& p, bool one_set)
     while (zs > 1 && chunks * ((c.nz + zs - 1) / zs) < (half ? 1000 : 10000) * zs) zs /= 2;
     t.zseg_interior = zs;
     t.zseg_slab = zs;
-    if (!one_set && c.block == 0) march_by_rule(p, t);
+    return t;
+}
+
+Tuning choose_tuning(const ShotPlan& p, bool one_set)
+{
+    Tuning t;
+    const ela3d_config& c = p.cfg;
+    const bool open = c.block == 0 && c.zseg == 0;
+    if (open && cached_tuning(c, t) && !(one_set && t.fused == 2)) return t;
+    t = two_pass_by_rule(p);
+    if (!one_set && open) march_by_rule(p, t);
+    return t;
+}
+
+// The shape of a live shot that goes on with two passes in place.  What is cached for its grid
+// by now may be of another schedule, whose second field set and stream the shot does not have.
+static Tuning in_place_tuning(const ShotPlan& p)
+{
+    Tuning t = choose_tuning(p, true);
+    if (t.fused) t = two_pass_by_rule(p);
+    t.dbuf = 0;
+    t.overlap = 0;
     return t;
 }
 
@@ -417,7 +435,7 @@ private:
             allocate();
         } catch (const Error& e) {  // no room for the second set of the whole-grid step
             if (e.code != ELA3D_E_OOM || sets_ != kSetAppended) throw;
-            tune_ = choose_tuning(plan_, true);
+            tune_ = in_place_tuning(plan_);
             set_shape(false);
             allocate();
         }
@@ -477,22 +495,22 @@ public:
     void enqueue_phase(int phase) override
     {
         HIP_CHECK(hipSetDevice(device_));
-        if (tune_.fused == 2 && sets_ == kSetAppended) leave_second_set();
-        if (tune_.fused || dbuf_ || overlap_)
+        const bool leave = tune_.fused == 2 && sets_ == kSetAppended;
+        if (overlap_ || (!leave && (tune_.fused || dbuf_)))
             throw Error{ELA3D_E_STATE, "stepping by phases needs the in-place two-pass schedule"};
+        if (phase != 0 && phase != 1) throw Error{ELA3D_E_INVALID, "phase must be 0 (stress pass) or 1 (velocity pass and tail)"};
+        if (leave) leave_second_set();
         const int it = host_step_ + 1;
         const bool e = energy_step(it);
         if (phase == 0) {
             launch_stress(args_[0][1][0], stream_);
             launch_stress(args_[0][0][0], stream_);
-        } else if (phase == 1) {
+        } else {
             launch_velocity(args_[0][1][1], e, stream_);
             launch_velocity(args_[0][0][1], e, stream_);
             if (e) launch_epart(d_epart_, nepart_, d_epart2_, epart_blocks(), stream_);
             launch_tail(tail_args(0), stream_);
             step_enqueued(it);
-        } else {
-            throw Error{ELA3D_E_INVALID, "phase must be 0 (stress pass) or 1 (velocity pass and tail)"};
         }
         HIP_CHECK(hipGetLastError());
     }
@@ -518,8 +536,9 @@ public:
     // From the whole-grid step to two passes in place, for calls that only those serve.  The second set stays allocated, unused.
     void leave_second_set()
     {
+        const Tuning t = in_place_tuning(plan_);
         to_first_set();
-        tune_ = choose_tuning(plan_, true);
+        tune_ = t;
         dbuf_ = false;
         for (int q = 0; q < 9; ++q) d_f_[1][q] = d_f_[0][q];
         for (int q = 0; q < 18; ++q) d_m_[1][q] = d_m_[0][q];

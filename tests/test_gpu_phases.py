@@ -1,0 +1,45 @@
+"""GPU: stepping by phases a shot that was created with the whole-grid step."""
+import numpy as np
+import pytest
+
+from ela3d_amd import SRC_EXPLOSIVE, STORAGE_FP32, STORAGE_FP64, Ela3dError, Shot, set_tuning
+from helpers import hetero_model, small_cfg
+
+pytestmark = pytest.mark.gpu
+E_INVALID = -1
+
+
+def fields(shot):
+    return [shot.snapshot(q) for q in range(27)]
+
+
+#                    nx  ny  nz   what is cached for the grid once the shot is there
+@pytest.mark.parametrize("dims,later", [
+    ((46, 47, 28), dict(fused=1, tile=512)), ((47, 46, 28), dict(fused=1, tile=512, overlap=True)),
+    ((48, 45, 28), dict(overlap=True)), ((45, 48, 28), dict(dbuf=True, merged=True)),
+    ((44, 49, 28), dict(fused=2, tile=320))])
+@pytest.mark.parametrize("storage", [STORAGE_FP32, STORAGE_FP64])
+def test_grid_tuned_after_the_shot_was_created(gpu, dims, later, storage):
+    """Phases go on in place with two passes whatever the grid was tuned to meanwhile, and the
+    steps after them give the same fields bit for bit; a refused phase leaves the shot as it is."""
+    cfg = small_cfg(nx=dims[0], ny=dims[1], nz=dims[2], nstep=23, storage=storage, src_kind=SRC_EXPLOSIVE,
+                    energy_every=0)
+    model = hetero_model(cfg, seed=6)
+    with Shot(cfg.replace(block=128, zseg=2), *model) as s:
+        s.run()
+        ref, seis = fields(s), s.seismograms()
+    with Shot(cfg, *model) as s:
+        assert s.info()["fused"] == 2
+        s.step(5)  # still running when the shot changes over
+        set_tuning(cfg, block=128, zseg_interior=4, zseg_slab=2, **later)
+        with pytest.raises(Ela3dError) as e:
+            s.step_phase(2)
+        assert e.value.code == E_INVALID and s.info()["fused"] == 2
+        for _ in range(3):
+            s.step_phase(0)
+            s.step_phase(1)
+        i = s.info()
+        assert (i["fused"], i["dbuf"], i["overlap"], i["steps_done"]) == (0, 0, 0, 8)
+        s.run()
+        assert np.array_equal(s.seismograms(), seis)
+        assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
