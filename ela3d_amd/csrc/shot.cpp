@@ -538,6 +538,7 @@ public:
     {
         const Tuning t = in_place_tuning(plan_);
         to_first_set();
+        HIP_CHECK(hipStreamSynchronize(stream_));  // the graphs destroyed below may still be running
         tune_ = t;
         dbuf_ = false;
         for (int q = 0; q < 9; ++q) d_f_[1][q] = d_f_[0][q];

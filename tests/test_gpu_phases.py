@@ -43,3 +43,20 @@ def test_grid_tuned_after_the_shot_was_created(gpu, dims, later, storage):
         s.run()
         assert np.array_equal(s.seismograms(), seis)
         assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
+
+
+def test_changes_over_with_graphs_in_flight(gpu):
+    """A phase asked for while hundreds of replayed steps are queued runs after them."""
+    cfg = small_cfg(nx=61, ny=43, nz=39, nstep=420, src_kind=SRC_EXPLOSIVE, energy_every=0)
+    model = hetero_model(cfg, seed=9)
+    with Shot(cfg.replace(block=128, zseg=2), *model) as s:
+        s.run()
+        ref, seis = fields(s), s.seismograms()
+    with Shot(cfg, *model) as s:
+        assert s.info()["fused"] == 2
+        s.step(401)
+        s.step_phase(0)
+        s.step_phase(1)
+        s.step(18)
+        assert np.array_equal(s.seismograms(), seis)
+        assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
