@@ -533,7 +533,7 @@ public:
         par_ = 0;
     }
 
-    // From the whole-grid step to two passes in place, for calls that only those serve.  The second set stays allocated, unused.
+    // From the whole-grid step to two passes in place, for calls that only those serve.
     void leave_second_set()
     {
         const Tuning t = in_place_tuning(plan_);
@@ -547,6 +547,35 @@ public:
         nepart_ = geo_[0].nblocks + geo_[1].nblocks;
         set_args();
         drop_graphs();
+        give_back_second_set();
+    }
+
+    // Everything before the second set moves to an allocation of its own size.  Where there is
+    // no room for that beside the old one, the second set stays allocated, unused.
+    void give_back_second_set()
+    {
+        if (mem_.arena) return;
+        const ArenaLayout L = arena_layout(plan_, int(sizeof(T)), nepart_, kOneSet);
+        if (int64_t(L.total) != state_bytes_) return;
+        void* one = nullptr;
+        try {
+            one = device_alloc(L.total);
+        } catch (const Error&) {
+            return;
+        }
+        try {
+            HIP_CHECK(hipMemcpyAsync(one, arena_, L.total, hipMemcpyDeviceToDevice, stream_));
+            HIP_CHECK(hipStreamSynchronize(stream_));
+        } catch (...) {
+            device_free(one, L.total);
+            throw;
+        }
+        device_free(arena_, size_t(arena_bytes_));
+        arena_ = one;
+        arena_bytes_ = int64_t(L.total);
+        sets_ = kOneSet;
+        place(L);
+        set_args();
     }
 
     // fields that cross a z interface after `phase`, sent towards higher k (up) or lower k
@@ -1064,6 +1093,36 @@ private:
                 }
     }
 
+    // the buffers' addresses in arena_
+    void place(const ArenaLayout& L)
+    {
+        char* b = static_cast<char*>(arena_);
+        for (int q = 0; q < 9; ++q) {
+            d_f_[0][q] = reinterpret_cast<T*>(b + L.f[q]) + guard_;
+            d_f_[1][q] = reinterpret_cast<T*>(b + L.f2[q]) + guard_;
+        }
+        for (int q = 0; q < 18; ++q) {
+            d_m_[0][q] = reinterpret_cast<T*>(b + L.m[q]);
+            d_m_[1][q] = reinterpret_cast<T*>(b + L.m2[q]);
+        }
+        for (int q = 0; q < 3; ++q) d_model_[q] = reinterpret_cast<float*>(b + L.model[q]) + guard_;
+        for (int q = 0; q < 3; ++q) d_tab_[q] = reinterpret_cast<double*>(b + L.tab[q]);
+        d_wav_ = reinterpret_cast<double*>(b + L.wav);
+        d_rec_ = reinterpret_cast<int*>(b + L.rec);
+        d_seis_ = reinterpret_cast<double*>(b + L.seis);
+        d_energy_ = reinterpret_cast<double*>(b + L.energy);
+        d_epart_ = reinterpret_cast<double*>(b + L.epart);
+        d_epart2_ = reinterpret_cast<double*>(b + L.epart2);
+        d_step_ = reinterpret_cast<int*>(b + L.ctl);
+        d_flag_ = d_step_ + 1;
+        d_presrc_ = reinterpret_cast<double*>(d_step_ + 4);
+        d_scl_ = reinterpret_cast<float*>(b + L.scl);
+        d_maxslot_ = reinterpret_cast<unsigned*>(b + L.slot);
+        d_srctrace_ = reinterpret_cast<double*>(b + L.srctrace);
+        d_tabf_ = reinterpret_cast<float*>(b + L.tabf);
+        d_side_ = reinterpret_cast<float*>(b + L.side);
+    }
+
     void allocate()
     {
         const ela3d_config& c = plan_.cfg;
@@ -1073,12 +1132,6 @@ private:
         const ArenaLayout L = arena_layout(plan_, int(sizeof(T)), nepart_, sets_);
         epart_cap_ = L.epart_cap;
         const size_t off = L.total;
-        const size_t* o_f = L.f;
-        const size_t* o_m = L.m;
-        const size_t* o_model = L.model;
-        const size_t* o_tab = L.tab;
-        const size_t o_wav = L.wav, o_rec = L.rec, o_seis = L.seis, o_en = L.energy, o_ep = L.epart;
-        const size_t o_ctl = L.ctl, o_scl = L.scl, o_slot = L.slot, o_src = L.srctrace;
         arena_bytes_ = int64_t(off);
         state_bytes_ = int64_t(L.state);
         if (mem_.arena) {
@@ -1089,31 +1142,7 @@ private:
         } else {
             arena_ = device_alloc(off);
         }
-        char* b = static_cast<char*>(arena_);
-        for (int q = 0; q < 9; ++q) {
-            d_f_[0][q] = reinterpret_cast<T*>(b + o_f[q]) + guard_;
-            d_f_[1][q] = reinterpret_cast<T*>(b + L.f2[q]) + guard_;
-        }
-        for (int q = 0; q < 18; ++q) {
-            d_m_[0][q] = reinterpret_cast<T*>(b + o_m[q]);
-            d_m_[1][q] = reinterpret_cast<T*>(b + L.m2[q]);
-        }
-        for (int q = 0; q < 3; ++q) d_model_[q] = reinterpret_cast<float*>(b + o_model[q]) + guard_;
-        for (int q = 0; q < 3; ++q) d_tab_[q] = reinterpret_cast<double*>(b + o_tab[q]);
-        d_wav_ = reinterpret_cast<double*>(b + o_wav);
-        d_rec_ = reinterpret_cast<int*>(b + o_rec);
-        d_seis_ = reinterpret_cast<double*>(b + o_seis);
-        d_energy_ = reinterpret_cast<double*>(b + o_en);
-        d_epart_ = reinterpret_cast<double*>(b + o_ep);
-        d_epart2_ = reinterpret_cast<double*>(b + L.epart2);
-        d_step_ = reinterpret_cast<int*>(b + o_ctl);
-        d_flag_ = d_step_ + 1;
-        d_presrc_ = reinterpret_cast<double*>(d_step_ + 4);
-        d_scl_ = reinterpret_cast<float*>(b + o_scl);
-        d_maxslot_ = reinterpret_cast<unsigned*>(b + o_slot);
-        d_srctrace_ = reinterpret_cast<double*>(b + o_src);
-        d_tabf_ = reinterpret_cast<float*>(b + L.tabf);
-        d_side_ = reinterpret_cast<float*>(b + L.side);
+        place(L);
         // zero everything: wavefields and memory variables (CPU:107-140), the guards
         // and plane padding (read as neighbours, never written), outputs
         if (mem_.arena) {  // memory the shot does not own may hold a previous user's data

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from ela3d_amd import SRC_EXPLOSIVE, STORAGE_FP32, STORAGE_FP64, Ela3dError, Shot, set_tuning
+from ela3d_amd import SRC_EXPLOSIVE, STORAGE_FP32, STORAGE_FP64, Ela3dError, Shot, set_device_limit, set_tuning
 from helpers import hetero_model, small_cfg
 
 pytestmark = pytest.mark.gpu
@@ -59,4 +59,31 @@ def test_changes_over_with_graphs_in_flight(gpu):
         s.step_phase(1)
         s.step(18)
         assert np.array_equal(s.seismograms(), seis)
+        assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
+
+
+@pytest.mark.parametrize("storage", [STORAGE_FP32, STORAGE_FP64])
+@pytest.mark.parametrize("room", [True, False])
+def test_second_field_set_is_given_back(gpu, storage, room):
+    """A shot that steps by phases needs one field set and holds no more than that, except where
+    there is no room to move it; either way it goes on bit for bit, checkpoints included."""
+    cfg = small_cfg(nx=63, ny=31, nz=29, nstep=24, storage=storage, src_kind=SRC_EXPLOSIVE, energy_every=3)
+    model = hetero_model(cfg, seed=10)
+    with Shot(cfg.replace(block=128, zseg=2), *model) as s:
+        one = s.info()["device_bytes"]
+        s.run()
+        ref, seis, trace = fields(s), s.seismograms(), s.source_trace()
+    with Shot(cfg, *model) as s:
+        two = s.info()["device_bytes"]
+        assert s.info()["fused"] == 2 and two > one
+        s.step(3)
+        try:
+            set_device_limit(0 if room else two + one - 1)
+            s.step_phase(0)
+            s.step_phase(1)
+        finally:
+            set_device_limit(0)
+        assert s.info()["device_bytes"] == (one if room else two)
+        s.run()
+        assert np.array_equal(s.seismograms(), seis) and np.array_equal(s.source_trace(), trace)
         assert all(np.array_equal(x, y) for x, y in zip(ref, fields(s)))
