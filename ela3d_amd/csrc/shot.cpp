@@ -12,6 +12,7 @@
 //   [nsamples][nrec][3], energy [nenergy][2], energy partials.
 #include "shot.hpp"
 #include "geom.hpp"
+#include "runs.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -398,6 +399,7 @@ public:
         plan_ = std::move(plan);
         mem_ = mem;
         const ela3d_config& c = plan_.cfg;
+        runs_.set_energy(c.energy_every);
         HIP_CHECK(hipSetDevice(c.device));
         device_ = c.device;
         try {
@@ -465,9 +467,7 @@ private:
         (void)hipSetDevice(device_);
         if (stream_ || mem_.arena) (void)hipStreamSynchronize(stream_);
         if (aux_) (void)hipStreamSynchronize(aux_);
-        for (auto& g : graphs_)
-            if (g.exec) (void)hipGraphExecDestroy(g.exec);
-        graphs_.clear();
+        drop_graphs();
         if (arena_ && !mem_.arena) device_free(arena_, size_t(arena_bytes_));
         if (h_flag_ && h_flag_ != mem_.host_flag) (void)hipHostFree(h_flag_);
         if (aux_) (void)hipStreamDestroy(aux_);
@@ -644,70 +644,38 @@ public:
         if (sets_ == kSetAppended && dbuf_) to_first_set();
     }
 
-    // One graph holds a run of consecutive steps: between two graphs the GPU idles for 4 to 8 us
-    // (64^3, kernels 19 us a step: 24 us with one step per graph, 20 with 16), a graph's own
-    // nodes follow each other at once.  Runs are up to 16 steps, where the gap has become small,
-    // and whole energy cycles where those are shorter, so that a long run repeats one graph.
-    // Capturing costs about 5 us a step, what its gaps cost once: a run is captured when it
-    // comes up for the second time, and made of single steps before.
-    static constexpr int kGraphSteps = 16;
-    static constexpr size_t kGraphs = 16;
+    // the next n steps as a run (see runs.hpp)
+    StepRun next_run(int n) const
+    {
+        StepRun r{cur(), n, 0};
+        for (int s = 0; s < n; ++s) r.energy |= unsigned(energy_step(host_step_ + 1 + s)) << s;
+        return r;
+    }
 
-    // n steps (0 < n <= graph_steps()) the production way: replays of captured graphs, or eager
+    // n steps, a run or a part of one, the production way: replays of captured graphs, or eager
     // launches when graphs are off
     void graph_run(int n)
     {
-        const int par = cur();
-        unsigned energy = 0;  // bit s: step s of the run sums the energy
-        for (int s = 0; s < n; ++s) energy |= unsigned(energy_step(host_step_ + 1 + s)) << s;
+        const StepRun r = next_run(n);
         if (!plan_.cfg.use_graph) {
-            launch_run(n, energy, par);
-        } else if (StepGraph& g = graph_of(n, energy, par); g.exec) {
-            HIP_CHECK(hipGraphLaunch(g.exec, stream_));
+            launch_run(n, r.energy, r.par);
+        } else if (hipGraphExec_t g = runs_.graph(r, [&] { return capture(n, r.energy, r.par); })) {
+            HIP_CHECK(hipGraphLaunch(g, stream_));
         } else {
-            for (int s = 0; s < n; ++s) graph_run(1);
+            runs_.parts(r, [&](int part) { graph_run(part); });
             return;
         }
         for (int s = 0; s < n; ++s) step_enqueued(host_step_ + 1);
-    }
-    // the cache's entry for a run, made the most recent; captured unless it is a longer run seen
-    // for the first time
-    struct StepGraph {
-        int par, steps;
-        unsigned energy;
-        hipGraphExec_t exec;
-    };
-    StepGraph& graph_of(int n, unsigned energy, int par)
-    {
-        auto it = std::find_if(graphs_.begin(), graphs_.end(), [&](const StepGraph& g) {
-            return g.par == par && g.steps == n && g.energy == energy;
-        });
-        if (it != graphs_.end()) {
-            std::rotate(it, it + 1, graphs_.end());
-        } else {
-            if (graphs_.size() == kGraphs) {  // the least recently used one may still be running
-                HIP_CHECK(hipStreamSynchronize(stream_));
-                if (graphs_.front().exec) (void)hipGraphExecDestroy(graphs_.front().exec);
-                graphs_.erase(graphs_.begin());
-            }
-            graphs_.push_back(StepGraph{par, n, energy, nullptr});
-            if (n > 1) return graphs_.back();
-        }
-        StepGraph& g = graphs_.back();
-        if (!g.exec) g.exec = capture(n, energy, par);
-        return g;
-    }
-    int graph_steps() const
-    {
-        const int ee = plan_.cfg.energy_every;
-        return ee > 0 && ee <= kGraphSteps ? kGraphSteps / ee * ee : kGraphSteps;
     }
 
     void enqueue_steps(int n) override
     {
         HIP_CHECK(hipSetDevice(device_));
-        const int run = graph_steps();
-        for (; n > 0; n -= run) graph_run(std::min(n, run));
+        while (n > 0) {
+            const int run = runs_.first(host_step_, n);
+            graph_run(run);
+            n -= run;
+        }
         HIP_CHECK(hipGetLastError());
     }
 
@@ -1015,9 +983,7 @@ public:
 
     void drop_graphs()
     {
-        for (auto& g : graphs_)
-            if (g.exec) (void)hipGraphExecDestroy(g.exec);
-        graphs_.clear();
+        runs_.clear([](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
     }
 
     void info(ela3d_info& o) override
@@ -1500,7 +1466,7 @@ private:
             launch_step(energy >> s & 1u, nullptr, dbuf_ ? (par + s) & 1 : 0, s > 0, s == n - 1);
     }
 
-    // the run of graph_run as a graph; a capture that fails leaves the stream out of capture
+    // a run as a graph; a capture that fails leaves the stream out of capture
     hipGraphExec_t capture(int n, unsigned energy, int par)
     {
         hipGraph_t graph = nullptr;
@@ -1624,8 +1590,7 @@ private:
         HIP_CHECK(hipMemcpy(d_scl_ + 108 + q, &m, sizeof(float), hipMemcpyHostToDevice));
         return sc;
     }
-    // runs of steps, least recently used first
-    std::vector<StepGraph> graphs_;
+    StepRuns<hipGraphExec_t> runs_;
 };
 
 std::unique_ptr<Shot> make_shot(ShotPlan plan, const float* cp, const float* cs, const float* rho,
