@@ -63,6 +63,25 @@ void device_free(void* p, size_t bytes)
 // Last-level cache in front of HBM
 constexpr int64_t kInfinityCache = int64_t(256) << 20;
 
+static size_t mem_elems(const ShotPlan& p, int axis)
+{
+    const ela3d_config& c = p.cfg;
+    const PmlAxis& A = p.ax[axis];
+    if (axis == 0) return size_t(c.nz) * c.ny * A.width();
+    if (axis == 1) return size_t(c.nz) * A.width() * c.nx;
+    return size_t(A.width()) * c.ny * c.nx;
+}
+
+// Bytes of the arrays a step reads and writes: fields and memory variables, `sets` times, and
+// the model (not what a shot records, which a step hardly touches).
+static int64_t step_bytes(const ShotPlan& p, int sets)
+{
+    const int64_t cells = plane_stride(p.cfg.nx, p.cfg.ny) * p.cfg.nz;
+    int64_t state = 9 * cells;
+    for (int axis : kMemAxis) state += int64_t(mem_elems(p, axis));
+    return sets * state * storage_bytes(p.cfg.storage) + 3 * cells * int64_t(sizeof(float));
+}
+
 // The whole-grid fused step (march.hip) as the schedule of a new shot, in place of two passes.
 // It reads and writes every array once per step (two passes: about 1.6 times the bytes) but
 // keeps two field sets and, with few columns per wave, idles lanes.  Measured, us per step,
@@ -114,9 +133,7 @@ static bool march_by_rule(const ShotPlan& p, Tuning& t)
     m.zseg_interior = z;
     if (!march_unsupported(p, m).empty()) return false;
     if (tiles * ((c.nz + z - 1) / z) > fit && c.nx * 10 < xch * 64 * 6) return false;
-    const int elem = storage_bytes(c.storage);
-    const int64_t one = int64_t(arena_layout(p, elem, 0, kOneSet).total);
-    const int64_t two = int64_t(arena_layout(p, elem, 0, kSetAppended).total);
+    const int64_t one = step_bytes(p, 1), two = step_bytes(p, 2);
     if (two > (int64_t(16) << 30)) return false;
     if (two > kInfinityCache && one <= kInfinityCache) return false;
     t = m;
@@ -312,15 +329,6 @@ std::string march_unsupported(const ShotPlan& p, const Tuning& t)
     return "";
 }
 
-static size_t mem_elems(const ShotPlan& p, int axis)
-{
-    const ela3d_config& c = p.cfg;
-    const PmlAxis& A = p.ax[axis];
-    if (axis == 0) return size_t(c.nz) * c.ny * A.width();
-    if (axis == 1) return size_t(c.nz) * A.width() * c.nx;
-    return size_t(A.width()) * c.ny * c.nx;
-}
-
 // Byte offsets of every buffer in a shot's single device allocation.  Each
 // buffer starts on a 256-byte boundary; the energy-partial buffer has room for
 // any launch shape the tuner may pick (block >= 64, vec >= 1, zseg >= 1).
@@ -444,12 +452,6 @@ private:
         upload(cp, cs, rho);
         initial_scales(cp, rho);
         set_args();
-    }
-
-    // bytes of the arrays a step reads and writes
-    int64_t state_moved() const
-    {
-        return int64_t(arena_layout(plan_, int(sizeof(T)), 0, dbuf_ ? kSetAppended : kOneSet).total);
     }
 
     // sets, overlap and geometry of tune_
@@ -1290,7 +1292,8 @@ private:
         // the one before it touched last, still cached (one launch a step: 144^3 105 -> 99 us,
         // 160^3 134 -> 125, 201^3 244 -> 232; two passes: 201^3 256 -> 244, FP16 256^3 343 -> 336).
         // Larger grids and cached ones gain nothing and lose up to 1 %.
-        const bool turn = state_moved() > kInfinityCache && state_moved() <= 4 * kInfinityCache;
+        const int64_t moved = step_bytes(plan_, dbuf_ ? 2 : 1);
+        const bool turn = moved > kInfinityCache && moved <= 4 * kInfinityCache;
         a.back = !turn ? 0 : tune_.fused ? par : pass;
         a.xch = g.xch;
         a.xw = g.xw;
