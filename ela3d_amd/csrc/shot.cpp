@@ -63,23 +63,13 @@ void device_free(void* p, size_t bytes)
 // Last-level cache in front of HBM
 constexpr int64_t kInfinityCache = int64_t(256) << 20;
 
-static size_t mem_elems(const ShotPlan& p, int axis)
+// Bytes a step works on with these field sets: the allocation without the wavelet, the receivers
+// and what is recorded, of which a step touches a few lines (144^3, 4,000 steps, 1,000 receivers:
+// 96 of 272 MB).
+static int64_t step_bytes(const ShotPlan& p, Sets sets)
 {
-    const ela3d_config& c = p.cfg;
-    const PmlAxis& A = p.ax[axis];
-    if (axis == 0) return size_t(c.nz) * c.ny * A.width();
-    if (axis == 1) return size_t(c.nz) * A.width() * c.nx;
-    return size_t(A.width()) * c.ny * c.nx;
-}
-
-// Bytes of the arrays a step reads and writes: fields and memory variables, `sets` times, and
-// the model (not what a shot records, which a step hardly touches).
-static int64_t step_bytes(const ShotPlan& p, int sets)
-{
-    const int64_t cells = plane_stride(p.cfg.nx, p.cfg.ny) * p.cfg.nz;
-    int64_t state = 9 * cells;
-    for (int axis : kMemAxis) state += int64_t(mem_elems(p, axis));
-    return sets * state * storage_bytes(p.cfg.storage) + 3 * cells * int64_t(sizeof(float));
+    const ArenaLayout L = arena_layout(p, storage_bytes(p.cfg.storage), 0, sets);
+    return int64_t(L.total - (L.epart - L.wav) - (L.tabf - L.srctrace));
 }
 
 // The whole-grid fused step (march.hip) as the schedule of a new shot, in place of two passes.
@@ -133,7 +123,7 @@ static bool march_by_rule(const ShotPlan& p, Tuning& t)
     m.zseg_interior = z;
     if (!march_unsupported(p, m).empty()) return false;
     if (tiles * ((c.nz + z - 1) / z) > fit && c.nx * 10 < xch * 64 * 6) return false;
-    const int64_t one = step_bytes(p, 1), two = step_bytes(p, 2);
+    const int64_t one = step_bytes(p, kOneSet), two = step_bytes(p, kSetAppended);
     if (two > (int64_t(16) << 30)) return false;
     if (two > kInfinityCache && one <= kInfinityCache) return false;
     t = m;
@@ -327,6 +317,15 @@ std::string march_unsupported(const ShotPlan& p, const Tuning& t)
     // (a set of partials each for the step in progress and the one being recorded)
     if (2 * int64_t(all.nblocks) > epart_capacity(c)) return "too many workgroups for the energy partials";
     return "";
+}
+
+static size_t mem_elems(const ShotPlan& p, int axis)
+{
+    const ela3d_config& c = p.cfg;
+    const PmlAxis& A = p.ax[axis];
+    if (axis == 0) return size_t(c.nz) * c.ny * A.width();
+    if (axis == 1) return size_t(c.nz) * A.width() * c.nx;
+    return size_t(A.width()) * c.ny * c.nx;
 }
 
 // Byte offsets of every buffer in a shot's single device allocation.  Each
@@ -1292,7 +1291,7 @@ private:
         // the one before it touched last, still cached (one launch a step: 144^3 105 -> 99 us,
         // 160^3 134 -> 125, 201^3 244 -> 232; two passes: 201^3 256 -> 244, FP16 256^3 343 -> 336).
         // Larger grids and cached ones gain nothing and lose up to 1 %.
-        const int64_t moved = step_bytes(plan_, dbuf_ ? 2 : 1);
+        const int64_t moved = step_bytes(plan_, dbuf_ ? kSetAppended : kOneSet);
         const bool turn = moved > kInfinityCache && moved <= 4 * kInfinityCache;
         a.back = !turn ? 0 : tune_.fused ? par : pass;
         a.xch = g.xch;
