@@ -855,7 +855,7 @@ public:
                 const float v = float(in[sc_cell]);
                 HIP_CHECK(hipMemcpy(d_side_ + (field - 3), &v, sizeof(float), hipMemcpyHostToDevice));
             }
-            for (int b = 0; b < (dbuf_ ? 2 : 1); ++b)  // both sets: cells a step never writes keep it
+            for (int b = 0; b < (sets_ != kOneSet ? 2 : 1); ++b)  // both sets: cells a step never writes keep it
                 HIP_CHECK(hipMemcpy(d_f_[b][field], h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
             return;
         }
@@ -875,7 +875,7 @@ public:
                 throw Error{ELA3D_E_INVALID,
                             "memory variables are stored only inside the C-PML layers; "
                             "non-zero value outside them"};
-        for (int b = 0; b < (dbuf_ ? 2 : 1); ++b)
+        for (int b = 0; b < (sets_ != kOneSet ? 2 : 1); ++b)
             if (nm) HIP_CHECK(hipMemcpy(d_m_[b][m], h.data(), nm * sizeof(T), hipMemcpyHostToDevice));
     }
 
@@ -960,8 +960,8 @@ public:
             throw Error{ELA3D_E_INVALID, "the fused interior step needs both sets of an array side by side"};
         HIP_CHECK(hipSetDevice(device_));
         HIP_CHECK(hipStreamSynchronize(stream_));
-        if ((t.dbuf != 0 || t.fused != 0) && !dbuf_)
-            throw Error{ELA3D_E_INVALID, "double buffering is fixed when the shot is created"};
+        const bool two = t.dbuf != 0 || t.fused != 0;
+        if (two && sets_ == kOneSet) throw Error{ELA3D_E_INVALID, "this shot has one field set"};
         if (t.overlap != 0 && mem_.inplace) throw Error{ELA3D_E_INVALID, "this shot runs its launches in sequence"};
         if (t.fused) {
             const std::string why = t.fused == 2 ? march_unsupported(plan_, t) : fused_unsupported(plan_, t.tile);
@@ -971,6 +971,11 @@ public:
         geometry(plan_, t, g[1], g[0]);
         if (g[0].nblocks + g[1].nblocks > epart_cap_)
             throw Error{ELA3D_E_INVALID, "launch shape needs too many blocks"};
+        // two passes that do not ask for both sets update the first in place, as they will in
+        // a shot that has only one
+        if (dbuf_ && !two) to_first_set();
+        if (!dbuf_) par_ = 0;
+        dbuf_ = two;
         tune_ = t;
         tune_.dbuf = dbuf_ ? 1 : 0;
         overlap_ = t.overlap != 0;

@@ -81,7 +81,8 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
         ela3d::ShotPlan plan = ela3d::make_plan(c);
         int n = 0;
         if (hipGetDeviceCount(&n) != hipSuccess || n <= c.device) throw Error{ELA3D_E_NODEVICE, "no HIP device"};
-        // a second field set lets the scratch shot also try the fused schedules
+        // a second field set lets the scratch shot also try the fused schedules; its two-pass
+        // candidates update the first one in place, cached as they are in the shots they are for
         const bool fusable = ela3d::fused_unsupported(plan, 1024).empty() || ela3d::fused_unsupported(plan, 512).empty();
         Tuning whole;
         whole.fused = 2;
