@@ -392,7 +392,7 @@ private:
                 c.device = opts_.device;
                 return c;
             }());
-            const size_t need = size_t(shot_device_bytes(plan, r->one_set));
+            size_t need = size_t(shot_device_bytes(plan, r->one_set));
             for (size_t q = 0; q < slots_.size(); ++q)
                 if (!slots_[q].busy) {
                     r->slot = int(q);
@@ -401,7 +401,14 @@ private:
             if (r->slot < 0) throw Error{ELA3D_E_STATE, "no free stream slot"};
             Slot& sl = slots_[size_t(r->slot)];
             sl.busy = true;
-            r->mem = pool_.alloc(need);
+            try {
+                r->mem = pool_.alloc(need);
+            } catch (const Error& e) {  // no room for the whole-grid step's second set: as ela3d_create
+                if (e.code != ELA3D_E_OOM || r->one_set) throw;
+                r->one_set = true;
+                need = size_t(shot_device_bytes(plan, true));
+                r->mem = pool_.alloc(need);
+            }
             ShotMem mem;
             mem.arena = r->mem;
             mem.bytes = need;
