@@ -86,16 +86,6 @@ __device__ __forceinline__ R recur(R psi, R a, R b, R Kinv, R& d)
     return p;
 }
 
-// dt over the averaged density, to the rounding of the IEEE quotient: the hardware
-// reciprocal, and one Newton correction of the product's residual
-__device__ __forceinline__ float dt_quot(float dt, float r)
-{
-    const float y = __builtin_amdgcn_rcpf(r);
-    const float q = dt * y;
-    return __builtin_fmaf(__builtin_fmaf(-q, r, dt), y, q);
-}
-__device__ __forceinline__ double dt_quot(double dt, double r) { return dt / r; }
-
 // Cell energy terms of the total-energy sum, in the arithmetic type R (FP32
 // storage: FP32, about 1e-7 relative, below the state's own rounding; the sums
 // are FP64).  Kinetic 0.5 rho |v|^2.  Strain energy

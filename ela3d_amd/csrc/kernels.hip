@@ -194,14 +194,16 @@ __device__ __forceinline__ void stv(T* p, unsigned o, const typename Arith<T>::R
 
 // dt over the averaged density in the velocity updates: the reciprocal form
 // (dt_over) with FP16 storage, whose kernels are bound by instruction issue
-// (2.4-2.8 % faster on the layered grid); the corrected one with FP32 and FP64.
+// (2.4-2.8 % faster on the layered grid); the IEEE division with FP32 and FP64, whose
+// kernels wait for memory (a reciprocal and one correction measured the same within 0.4 %,
+// and gave NaN for densities below 1.2e-38).
 template <typename T, typename R>
 __device__ __forceinline__ R quot(R dt, R r)
 {
     if constexpr (std::is_same<T, half_t>::value)
         return dt_over(dt, r);
     else
-        return dt_quot(dt, r);
+        return dt / r;
 }
 
 // The updates' sums and products: written out with FP32 and FP64 (see sum_r); FP16 storage

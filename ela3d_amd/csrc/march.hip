@@ -506,7 +506,7 @@ struct Row {
             if constexpr (HASX) M.template xpml<false, GEN>(mv[0], on, d);
             d = add_axis<GEN>(d, sxy - r[-kSlot + kSxy * 64], idy, G.cy >= 0, on, my[0], G.Y);
             d = add_axis<GEN>(d, sxz - (surface ? -sxz : pxz), idz, G.cz >= 0, on, mz[0], G.Z);
-            const R v = fma_r(dt_quot(c[kCdtS * 64], (rhoc + rhoW) * (R)0.5), d, old);
+            const R v = fma_r(c[kCdtS * 64] / ((rhoc + rhoW) * (R)0.5), d, old);
             nvx = pick(free, GEN ? pick(on, v, old) : v, (R)0);
         }
         {  // vy (CPU:531-558)
@@ -516,7 +516,7 @@ struct Row {
             if constexpr (HASX) M.template xpml<true, GEN>(mv[1], on, d);
             d = add_axis<GEN>(d, r[kSlot + kSyy * 64] - r[kSyy * 64], idy, G.cy >= 0, on, my[1], G.Y + 3);
             d = add_axis<GEN>(d, syz - (surface ? -syz : below), idz, G.cz >= 0, on, mz[1], G.Z);
-            const R v = fma_r(dt_quot(c[kCdtN * 64], (rhoc + rhoN) * (R)0.5), d, old);
+            const R v = fma_r(c[kCdtN * 64] / ((rhoc + rhoN) * (R)0.5), d, old);
             nvy = pick(free, GEN ? pick(on, v, old) : v, (R)0);
         }
         {  // vz: the in-plane derivatives (CPU:562-590)
@@ -524,7 +524,7 @@ struct Row {
             R d = (east(sxz) - sxz) * idx;
             if constexpr (HASX) M.template xpml<true, GEN>(mv[2], on, d);
             hz = add_axis<GEN>(d, syz - r[-kSlot + kSyz * 64], idy, G.cy >= 0, on, my[2], G.Y);
-            hq = dt_quot(c[kCdtN * 64], (rhoc + rho) * (R)0.5);  // rho: of plane m+1 by now
+            hq = c[kCdtN * 64] / ((rhoc + rho) * (R)0.5);  // rho: of plane m+1 by now
             hs = szz;
             if (ENERGY) hr = rhoc;
         }
