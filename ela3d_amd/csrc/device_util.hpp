@@ -96,23 +96,38 @@ __device__ __forceinline__ R recur(R psi, R a, R b, R Kinv, R& d)
 // 1/(4 mu): FP32 holds the terms for stresses up to about 1e24 Pa (the unscaled
 // products s:s q overflow near 3e13 Pa, which the reference's own sigma source
 // parameters pass within a few dozen steps).
-template <typename R>
+// T: the storage; with FP16 the sums are left to the compiler, like the updates themselves.
+template <typename T, typename R>
 __device__ __forceinline__ R kinetic_energy(R rho, R vx, R vy, R vz)
 {
-    const R h = (R)0.5 * rho;
-    return fma_r(h * vx, vx, fma_r(h * vy, vy, (h * vz) * vz));
+    if constexpr (std::is_same<T, half_t>::value) {
+        return ((R)0.5 * rho * vx) * vx + ((R)0.5 * rho * vy) * vy + ((R)0.5 * rho * vz) * vz;
+    } else {
+        const R h = (R)0.5 * rho;
+        return fma_r(h * vx, vx, fma_r(h * vy, vy, (h * vz) * vz));
+    }
 }
-template <typename R>
+template <typename T, typename R>
 __device__ __forceinline__ R strain_energy(R rho, R vp, R vs, R sxx, R syy, R szz, R sxy, R sxz, R syz)
 {
-    const R mu = rho * vs * vs, lam = rho * fma_r(vp, vp, (R)-2 * vs * vs);
-    const R q = fma_r((R)3, lam, (R)2 * mu);
-    const R c = (R)1 / ((R)4 * mu * q);
-    const R a = q * c, a2 = (R)2 * a, b = lam * c;
-    const R tr = sxx + syy + szz;
-    const R n = fma_r(a * sxx, sxx, fma_r(a * syy, syy, (a * szz) * szz));
-    const R s = fma_r(a2 * sxy, sxy, fma_r(a2 * sxz, sxz, (a2 * syz) * syz));
-    return fma_r(-(b * tr), tr, n + s);
+    if constexpr (std::is_same<T, half_t>::value) {
+        const R mu = rho * vs * vs, lam = rho * (vp * vp - (R)2 * vs * vs);
+        const R q = (R)3 * lam + (R)2 * mu;
+        const R c = (R)1 / ((R)4 * mu * q);
+        const R a = q * c, a2 = (R)2 * a, b = lam * c;
+        const R tr = sxx + syy + szz;
+        return (a * sxx) * sxx + (a * syy) * syy + (a * szz) * szz +
+               (a2 * sxy) * sxy + (a2 * sxz) * sxz + (a2 * syz) * syz - (b * tr) * tr;
+    } else {
+        const R mu = rho * vs * vs, lam = rho * fma_r(vp, vp, (R)-2 * vs * vs);
+        const R q = fma_r((R)3, lam, (R)2 * mu);
+        const R c = (R)1 / ((R)4 * mu * q);
+        const R a = q * c, a2 = (R)2 * a, b = lam * c;
+        const R tr = sxx + syy + szz;
+        const R n = fma_r(a * sxx, sxx, fma_r(a * syy, syy, (a * szz) * szz));
+        const R s = fma_r(a2 * sxy, sxy, fma_r(a2 * sxz, sxz, (a2 * syz) * syz));
+        return fma_r(-(b * tr), tr, n + s);
+    }
 }
 
 // Streaming (nontemporal) store of element o of p.  For the nine wave fields: a

@@ -404,8 +404,8 @@ k_fused(const StepArgs<T> A)
             if (iN || face) stn(fw[2], oo, nvz);
             if (ENERGY) {
                 if (in_e_xy && k >= A.ek0 && k < A.ek1) {
-                    ek += kinetic_energy(S.rho, nvx, nvy, nvz);
-                    ep += strain_energy(S.rho, S.cp, S.cs, sxx, syy, S.szz, sxy, sxz, syz);
+                    ek += kinetic_energy<T>(S.rho, nvx, nvy, nvz);
+                    ep += strain_energy<T>(S.rho, S.cp, S.cs, sxx, syy, S.szz, sxy, sxz, syz);
                 }
             }
             pv_sxz = sxz;

@@ -825,8 +825,8 @@ __device__ __forceinline__ void velocity_update(const StepArgs<T>& A, const Lane
                               k < A.ek1;
             if (in_e) {
                 // state after this velocity update, cell-local: kinetic and strain energy
-                ek += (double)kinetic_energy(Q.rho_c[e], nvx[e], nvy[e], nvz[e]);
-                ep += (double)strain_energy(Q.rho_c[e], P.cp[e], P.cs[e], P.sxx[e], P.syy[e], Q.szz_c[e],
+                ek += (double)kinetic_energy<T>(Q.rho_c[e], nvx[e], nvy[e], nvz[e]);
+                ep += (double)strain_energy<T>(Q.rho_c[e], P.cp[e], P.cs[e], P.sxx[e], P.syy[e], Q.szz_c[e],
                                             P.sxy[e], P.sxz[e], P.syz[e]);
             }
         }

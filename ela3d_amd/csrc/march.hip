@@ -554,8 +554,8 @@ struct Row {
         }
         if constexpr (ENERGY) {
             const unsigned in = in_box(m);
-            const R k2 = kinetic_energy(rhoc, nvx, nvy, (R)0);
-            const R p2 = strain_energy(rhoc, cpc, (R)r[kUcs * 64], sxx, (R)r[kSyy * 64], szz, sxy, sxz, syz);
+            const R k2 = kinetic_energy<T>(rhoc, nvx, nvy, (R)0);
+            const R p2 = strain_energy<T>(rhoc, cpc, (R)r[kUcs * 64], sxx, (R)r[kSyy * 64], szz, sxy, sxz, syz);
             ek += (double)pick(in, k2, (R)0);
             ep += (double)pick(in, p2, (R)0);
         }
