@@ -75,7 +75,7 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
         c.nrec = 0;
         c.rec = nullptr;
         c.use_graph = 0;
-        c.nstep = std::max(c.nstep, steps * 64 + 16);
+        c.nstep = std::max(c.nstep, steps * 256 + 8192);  // energy steps come to the last candidate
         c.block = 256;
         c.zseg = 0;
         ela3d::ShotPlan plan = ela3d::make_plan(c);
@@ -209,15 +209,37 @@ int ela3d_autotune(const ela3d_config* cfg, const float* cp, const float* cs, co
             }
         }
         // schedule: the two launches in sequence, overlapped (pays off when neither
-        // fills the GPU), or one mixed launch per pass (one kernel boundary less)
+        // fills the GPU), or one mixed launch per pass (one kernel boundary less).
+        // Timed as steps one after the other between two events: events around every launch
+        // cost more than a small grid's kernels, the same for every schedule, and hid what
+        // its launches and their gaps take.  Long enough to last milliseconds, and
+        // whole energy cycles where those are short.
+        struct Events {
+            hipEvent_t at[2] = {nullptr, nullptr};
+            ~Events()
+            {
+                for (auto& e : at)
+                    if (e) (void)hipEventDestroy(e);
+            }
+        } ev;
+        for (auto& e : ev.at) HIP_CHECK(hipEventCreate(&e));
+        int n_wall = steps;
         auto wall_of = [&](const Tuning& t) {
             shot->retune(t);
-            double wall = 0.0;
-            shot->profile(1, st, wall);
-            shot->profile(steps, st, wall);
+            shot->enqueue_steps(std::max(1, n_wall / 8));
+            (void)shot->sync();
+            HIP_CHECK(hipEventRecord(ev.at[0], shot->stream()));
+            shot->enqueue_steps(n_wall);
+            HIP_CHECK(hipEventRecord(ev.at[1], shot->stream()));
+            HIP_CHECK(hipEventSynchronize(ev.at[1]));
+            float wall = 0.f;
+            HIP_CHECK(hipEventElapsedTime(&wall, ev.at[0], ev.at[1]));
             ++tried;
-            return wall / steps;
+            return double(wall) / n_wall;
         };
+        if (wall_of(best) < 0.3) n_wall = std::max(steps, 48);
+        if (c.energy_every > 0 && c.energy_every <= 16)
+            n_wall = (n_wall + c.energy_every - 1) / c.energy_every * c.energy_every;
         double wall3[3] = {0.0, 0.0, 1e300};
         Tuning cand[3] = {best, best, best};
         cand[1].overlap = 1;
