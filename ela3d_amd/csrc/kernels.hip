@@ -194,9 +194,8 @@ __device__ __forceinline__ void stv(T* p, unsigned o, const typename Arith<T>::R
 
 // dt over the averaged density in the velocity updates: the reciprocal form
 // (dt_over) with FP16 storage, whose kernels are bound by instruction issue
-// (2.4-2.8 % faster on the layered grid); the IEEE division with FP32 and FP64, whose
-// kernels wait for memory (a reciprocal and one correction measured the same within 0.4 %,
-// and gave NaN for densities below 1.2e-38).
+// (2.4-2.8 % faster on the layered grid); the IEEE division with FP32 and FP64
+// storage, where the reciprocal measured no faster in these kernels.
 template <typename T, typename R>
 __device__ __forceinline__ R quot(R dt, R r)
 {

@@ -144,7 +144,7 @@ void launch_fused(const StepArgs<T>& a, bool energy, hipStream_t s);
 template <typename T>
 size_t fused_lds_bytes(int nx, int tile);
 // fused step over the whole grid, absorbing layers included (march.hip); needs
-// double-buffered fields.  A workgroup has a wave per own row and two halo waves.
+// double-buffered fields.  A workgroup has a wave per own row and one for both halo rows.
 template <typename T>
 void launch_march(const StepArgs<T>& a, const TailArgs<T>& tail, bool energy, hipStream_t s);
 // records the last step of a run of them (`block` threads, as the step's workgroups)

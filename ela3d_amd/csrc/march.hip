@@ -16,6 +16,9 @@
 // streaming loads or stores were 5 to 30 % slower at 401 x 401 x 301, the next plane's loads
 // issued before the barrier (73 registers for 67) 2 %, 32 waves (spills) 5 %.  The halo rows
 // share a wave: one each would be idle for half a plane (101^3: 47 -> 41 us a step).
+// dt over the averaged densities is the IEEE division, for every density that is accepted: the
+// hardware reciprocal and one correction saved 0.1 to 0.4 us of a step of 33^3 to 113x97x85 and
+// nothing from 201^3 on, but gave NaN below 1.2e-38.
 //
 // Time per step, FP32, two passes of two launches and a tail against this: 33^3 19 -> 10 us,
 // 64^3 23 -> 15, 101^3 43 -> 35, 201^3 244 -> 228, 401x401x301 1305 -> 1173, 480x500x360
@@ -744,7 +747,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) 
         const int nb = M.ke - M.kb + (M.kb > 0 ? 2 : 1);
         for (int q = 0; q < nb; ++q) lds_barrier();
     }
-    if constexpr (ENERGY) {  // per-block FP64 partials, summed in block order by the tail kernel
+    if constexpr (ENERGY) {  // per-block FP64 partials, summed by whoever records the step (record_step)
         __shared__ double red[2][NT / 64];
         ek = wave_sum(ek);
         ep = wave_sum(ep);

@@ -112,7 +112,8 @@ public:
     // per-launch totals), the others graph replays; wall_ms spans all n
     virtual void profile(int n, std::vector<ela3d_kernel_stats>& st, double& wall_ms, int every = 1) = 0;
     virtual void info(ela3d_info& out) = 0;
-    virtual void retune(const Tuning& t) = 0;       // new launch shape (drops captured graphs)
+    // new launch shape (drops captured graphs); two passes without dbuf update the first set in place
+    virtual void retune(const Tuning& t) = 0;
     virtual hipStream_t stream() const = 0;
     // run the absorbing-layer launches concurrently with the interior ones (default)
     // or in sequence on the main stream (drops captured graphs)

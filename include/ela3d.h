@@ -116,7 +116,7 @@ typedef struct ela3d_config {
     int32_t dirichlet;      /* 1: vx=vy=vz=0 on the six faces after each velocity update */
     int32_t fp16_rescale_every; /* FP16 storage: re-choose scales every N steps (default 100) */
     int32_t device;         /* HIP device ordinal */
-    int32_t use_graph;      /* 1 (default): replay hipGraphs of up to 16 steps */
+    int32_t use_graph;      /* 1 (default): replay hipGraphs of runs of about 16 steps */
     int32_t block;          /* threads per workgroup, 0 = autotuned */
     int32_t zseg;           /* z planes per workgroup, 0 = autotuned */
     int32_t free_surface;   /* 1: traction-free surface at the plane k = 0 (no z-min C-PML
@@ -215,7 +215,8 @@ int ela3d_checkpoint_load(ela3d_shot* shot, const char* path);
 int ela3d_create_slab(const ela3d_config* cfg, int32_t k0, int32_t k1, const float* cp, const float* cs,
                       const float* rho, ela3d_shot** out, int32_t* receivers, size_t receivers_cap,
                       int32_t* nreceivers);
-/* phase 0: the stress pass; phase 1: the velocity pass, receivers, energy, source (one step) */
+/* phase 0: the stress pass; phase 1: the velocity pass, receivers, energy, source (one step).  A shot
+ * that runs the whole-grid step goes over to two passes in place with its first phase. */
 int ela3d_step_phase(ela3d_shot* shot, int32_t phase);
 /* bytes a halo_pack(phase, side) writes (what the neighbour's unpack on the other side reads) */
 int ela3d_halo_bytes(ela3d_shot* shot, int32_t phase, int32_t side, size_t* bytes);
